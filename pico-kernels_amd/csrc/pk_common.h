@@ -90,6 +90,13 @@ __device__ __forceinline__ float round_to_dtype(float v, int dtype) {
   return v;
 }
 
+// v as an fp32 result of its own. A product converted to fp16 right after is otherwise selected
+// as one v_fma_mixlo_f16 (a * b + 0): rounded once instead of twice, and -0 becomes +0.
+__device__ __forceinline__ float fp32_value(float v) {
+  asm("" : "+v"(v));
+  return v;
+}
+
 __device__ __forceinline__ void store_from_f32(void* p, int dtype, int64_t i, float v) {
   if (dtype == PK_F32) reinterpret_cast<float*>(p)[i] = v;
   else if (dtype == PK_F16) reinterpret_cast<pk_half*>(p)[i] = (pk_half)v;

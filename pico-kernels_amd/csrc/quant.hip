@@ -143,60 +143,306 @@ __global__ __launch_bounds__(kThreads) void unpack_int4_kernel(const uint8_t* __
 }
 
 // ---------------------------------------------------------------------------------------
-// Group RTN quantization along K (quantize.py:42-68).
+// Group RTN quantization along K (quantize.py:42-68): per column and group of rows the absmax,
+// the scale, then every row's code.
 //
-// One thread owns CPT consecutive columns of one group of rows. Pass 1 takes the group
-// absmax per column, pass 2 quantizes (the group re-read hits L1/L2). With CPT == 8 and
-// bits == 4 the thread emits whole 32-bit words of the packed (K, N/8) layout.
+// Bound by HBM (the weights in, codes and scales out). A thread owns 8 consecutive columns
+// (one word of the packed (K, N/8) layout, one or two 16-byte loads a row) of every RS-th row
+// of a group. Groups of at most 128 rows (quantize_group_kernel) are read once: 256 threads
+// take 256 columns, a thread's 16 rows stay in registers with all their loads in flight,
+// the 8 row sets' maxima meet in LDS, and the codes are made from the registers. Measured on
+// MI355X, 4096 x 14336 fp16, group 128: 520 -> 37.7 us, 3.9 TB/s (one thread per 8 columns and group
+// before, which read each element by a 2-byte load, twice, in 224 workgroups); 4 or 16 row sets,
+// or 64, 128 or 512 columns, in a workgroup run 42-63 us. Longer groups
+// (quantize_group_long_kernel; one scale per column is one group of K rows) do not fit the
+// registers: 1024 threads take 64 columns, so that few columns still make many workgroups,
+// and read the group twice (6144 x 4096 bf16, one scale per column: 31.8 ms -> 87 us).
 // ---------------------------------------------------------------------------------------
-template <int CPT>
-__global__ __launch_bounds__(kThreads) void quantize_group_kernel(
-    const void* __restrict__ w, int dtype, int64_t K, int64_t N, int64_t ldw, int qmax,
-    int group, int half_math, uint32_t* __restrict__ qweight, void* __restrict__ scales,
-    int scale_dtype, void* __restrict__ fake, int fake_dtype) {
-  const int64_t nchunks = cdiv(N, CPT);
-  const int64_t ngroups = cdiv(K, group);
-  const int64_t item = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (item >= nchunks * ngroups) return;
-  const int64_t g = item / nchunks, chunk = item - g * nchunks;
-  const int64_t n0 = chunk * CPT, k0 = g * group;
-  const int64_t k1 = (k0 + group < K) ? k0 + group : K;
+template <int DT>
+struct QgRow {  // 8 columns of one row as loaded
+  pk_u4v w[DT == PK_F32 ? 2 : 1];
+  __device__ __forceinline__ float at(int c) const {
+    if constexpr (DT == PK_F32) return __builtin_bit_cast(float, (uint32_t)w[c >> 2][c & 3]);
+    const uint32_t u = w[0][c >> 1];
+    const uint16_t h = (uint16_t)((c & 1) ? u >> 16 : u);
+    if constexpr (DT == PK_F16) return (float)__builtin_bit_cast(pk_half, h);
+    else return bf16_to_f32(h);
+  }
+};
+
+// Maxima of 8 columns as |v|'s bit patterns, which order as the values do (NaN above infinity, so
+// that a NaN wins as torch's max lets it): two 16-bit columns per word, or one fp32 column.
+template <int DT>
+struct QgMax {
+  static constexpr int kWords = DT == PK_F32 ? 8 : 4;
+  uint32_t m[kWords];
+  __device__ __forceinline__ void clear() {
+#pragma unroll
+    for (auto& x : m) x = 0u;
+  }
+  __device__ __forceinline__ void take(int i, uint32_t bits) {
+    if constexpr (DT == PK_F32) {
+      m[i] = max(m[i], bits);
+    } else {
+      typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+      m[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, m[i]),
+                                                                    __builtin_bit_cast(u16x2, bits)));
+    }
+  }
+  __device__ __forceinline__ void take(const QgRow<DT>& r) {
+    constexpr uint32_t kAbs = DT == PK_F32 ? 0x7fffffffu : 0x7fff7fffu;
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) take(i, r.w[i >> 2][i & 3] & kAbs);
+  }
+  __device__ __forceinline__ float at(int c) const {
+    QgRow<DT> r;
+#pragma unroll
+    for (int i = 0; i < kWords; ++i) r.w[i >> 2][i & 3] = m[i];
+    return r.at(c);
+  }
+};
+
+struct QgParams {
+  const void* w;
+  int64_t K, N, ldw;
+  int qmax, group, half_math;
+  uint32_t* qweight;
+  void* scales;
+  int scale_dtype;
+  void* fake;
+  int fake_dtype;
+  int fake_vec;  // fake's 8 columns of a thread may be stored together
+};
+
+// Row k's 8 columns from n0; VEC: rows of whole, 16-byte aligned chunks. Columns past N read 0.
+// ONCE: the row is read once (but for the rare row that is emitted again).
+template <int DT, bool VEC, bool ONCE>
+__device__ __forceinline__ QgRow<DT> qg_load(const QgParams& p, int64_t k, int64_t n0) {
+  constexpr int ES = DT == PK_F32 ? 4 : 2;
+  QgRow<DT> r;
+  const char* src = reinterpret_cast<const char*>(p.w) + (k * p.ldw + n0) * ES;
+  if constexpr (VEC) {
+#pragma unroll
+    for (int i = 0; i < ES / 2; ++i)
+      r.w[i] = ONCE ? __builtin_nontemporal_load(reinterpret_cast<const pk_u4v*>(src) + i)
+                    : reinterpret_cast<const pk_u4v*>(src)[i];
+  } else {
+    uint32_t u[2 * ES];
+#pragma unroll
+    for (int i = 0; i < 2 * ES; ++i) u[i] = 0u;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      if (n0 + c >= p.N) continue;
+      if constexpr (DT == PK_F32) u[c] = reinterpret_cast<const uint32_t*>(src)[c];
+      else u[c >> 1] |= (uint32_t)reinterpret_cast<const uint16_t*>(src)[c] << (16 * (c & 1));
+    }
+#pragma unroll
+    for (int i = 0; i < ES / 2; ++i) r.w[i] = pk_u4v{u[4 * i], u[4 * i + 1], u[4 * i + 2], u[4 * i + 3]};
+  }
+  return r;
+}
+
+// The group's scales s[c] (stored by the threads with `store`) and what the codes need.
+struct QgScale {
+  float s[8], inv[8];
+  bool divide;  // take the true quotient of every element
+};
+template <int DT>
+__device__ __forceinline__ QgScale qg_scale(const QgParams& p, const QgMax<DT>& m, int mdt,
+                                            int64_t g, int64_t n0, bool store) {
   // In fp16/bf16 tensor math the 1e-12 floor is itself rounded to the tensor dtype
   // (it underflows to 0 in fp16).
-  const int mdt = half_math ? dtype : PK_F32;
   const float floor_v = round_to_dtype(1e-12f, mdt);
-  const float fq = (float)qmax;
+  QgScale q;
+  q.divide = p.half_math != 0;
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const float amax = m.at(c);
+    const float a = amax < floor_v ? floor_v : amax;  // clamp_min, NaN passes through
+    q.s[c] = round_to_dtype(a / (float)p.qmax, mdt);
+    q.inv[c] = 1.0f / q.s[c];
+    q.divide |= !(q.s[c] > 0x1p-100f && q.s[c] < 0x1p100f);  // 1 / s stays a normal number
+    if (store && p.scales != nullptr && n0 + c < p.N)
+      store_from_f32(p.scales, p.scale_dtype, g * p.N + n0 + c, q.s[c]);
+  }
+  return q;
+}
 
-  float s[CPT];
+// One row's codes (and fake-quantized values). The code is rint(fl(v / s)). With t = fl(v * fl(1 / s)),
+// |t - fl(v / s)| < |t| 2^-22, so rint(t) is the same unless t is that close to a half-integer;
+// only then (and for scales whose reciprocal is not a normal number, and in 16-bit tensor math,
+// where the quotient is rounded to the dtype first) the division has to be carried out: returns
+// whether this row needs that, for the caller to emit it again with DIVIDE (a rare second pass
+// over single rows, so that the division's code stands once and not beside every row's).
+// Without it |v / s| is at most qmax (1 + 2^-23), so no code needs clamping, and none is NaN.
+template <int DT, bool FAKE, bool DIVIDE>
+__device__ __forceinline__ bool qg_emit(const QgParams& p, const QgRow<DT>& row, const QgScale& q,
+                                        int mdt, int64_t k, int64_t n0) {
+#pragma clang fp contract(off)  // every product and quotient rounded by itself
+  float r[8];
+  float near = 0.0f;
+  uint32_t word = 0;
+  if constexpr (DIVIDE) {
+    const float fq = (float)p.qmax;
 #pragma unroll
-  for (int c = 0; c < CPT; ++c) s[c] = 0.0f;
-  for (int64_t k = k0; k < k1; ++k) {
-#pragma unroll
-    for (int c = 0; c < CPT; ++c)
-      if (n0 + c < N) s[c] = nanmax(s[c], __builtin_fabsf(load_as_f32(w, dtype, k * ldw + n0 + c)));
-  }
-#pragma unroll
-  for (int c = 0; c < CPT; ++c) {
-    float a = s[c] < floor_v ? floor_v : s[c];  // clamp_min, NaN passes through
-    s[c] = round_to_dtype(a / fq, mdt);
-    if (scales != nullptr && n0 + c < N) store_from_f32(scales, scale_dtype, g * N + n0 + c, s[c]);
-  }
-  for (int64_t k = k0; k < k1; ++k) {
-    uint32_t word = 0;
-#pragma unroll
-    for (int c = 0; c < CPT; ++c) {
-      if (n0 + c >= N) continue;
-      float v = load_as_f32(w, dtype, k * ldw + n0 + c);
-      float t = round_to_dtype(v / s[c], mdt);
-      float r = clamp_nan(__builtin_rintf(t), -fq, fq);
-      if (fake != nullptr) {
-        float f = round_to_dtype(r * s[c], mdt);
-        store_from_f32(fake, fake_dtype, k * N + n0 + c, f);
-      }
-      int code = (r == r) ? (int)r : 0;
-      word |= ((uint32_t)code & 0xfu) << (4 * c);
+    for (int c = 0; c < 8; ++c) {
+      r[c] = clamp_nan(__builtin_rintf(round_to_dtype(row.at(c) / q.s[c], mdt)), -fq, fq);
+      word |= ((r[c] == r[c]) ? (uint32_t)(int)r[c] & 0xfu : 0u) << (4 * c);
     }
-    if (CPT == 8 && qweight != nullptr) qweight[k * (N / 8) + chunk] = word;
+  } else {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float t = row.at(c) * q.inv[c];
+      r[c] = __builtin_rintf(t);
+      near = __builtin_fmaxf(near, __builtin_fmaf(__builtin_fabsf(t), 0x1p-21f, __builtin_fabsf(t - r[c])));
+      word |= ((uint32_t)(int)r[c] & 0xfu) << (4 * c);
+    }
+  }
+  if (p.qweight != nullptr) p.qweight[k * (p.N / 8) + (n0 >> 3)] = word;
+  if constexpr (FAKE) {
+    float f[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) f[c] = round_to_dtype(fp32_value(r[c] * q.s[c]), mdt);
+    if (p.fake_dtype == PK_F32) {
+      float* o = reinterpret_cast<float*>(p.fake) + k * p.N + n0;
+      if (p.fake_vec) {
+        *reinterpret_cast<pk_f4*>(o) = pk_f4{f[0], f[1], f[2], f[3]};
+        *reinterpret_cast<pk_f4*>(o + 4) = pk_f4{f[4], f[5], f[6], f[7]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          if (n0 + c < p.N) o[c] = f[c];
+      }
+    } else {
+      uint16_t h[8];
+      if (p.fake_dtype == PK_F16) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) h[c] = __builtin_bit_cast(uint16_t, (pk_half)f[c]);
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) h[c] = f32_to_bf16_rne(f[c]);
+      }
+      uint16_t* o = reinterpret_cast<uint16_t*>(p.fake) + k * p.N + n0;
+      if (p.fake_vec) {
+        *reinterpret_cast<pk_u4v*>(o) =
+            pk_u4v{h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16),
+                   h[4] | ((uint32_t)h[5] << 16), h[6] | ((uint32_t)h[7] << 16)};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+          if (n0 + c < p.N) o[c] = h[c];
+      }
+    }
+  }
+  return !DIVIDE && (q.divide || near > 0.5f);
+}
+
+constexpr int kQgRows = 128;  // rows of a group the register kernel holds
+constexpr int kQgSets = 8;    // its row sets
+constexpr int kQgLanes = 32;  // threads along a row, 8 columns each
+constexpr int kQgThreads = kQgLanes * kQgSets;
+
+template <int DT, bool VEC, bool FAKE>
+__global__ __launch_bounds__(kQgThreads) void quantize_group_kernel(QgParams p) {
+  constexpr int PER = kQgRows / kQgSets;
+  constexpr int W = QgMax<DT>::kWords;
+  __shared__ uint32_t red[kQgSets][kQgLanes * W];
+  const int t = threadIdx.x, set = t / kQgLanes, cl = t % kQgLanes;
+  const int64_t tiles = cdiv(p.N, 8 * kQgLanes), items = tiles * cdiv(p.K, p.group);
+  const int mdt = p.half_math ? DT : PK_F32;
+  for (int64_t b = blockIdx.x; b < items; b += gridDim.x) {
+    const int64_t g = b / tiles, n0 = ((b - g * tiles) * kQgLanes + cl) * 8, k0 = g * p.group;
+    const int rows = (int)min((int64_t)p.group, p.K - k0);
+    const bool cols = n0 < p.N;
+    QgRow<DT> v[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int r = i * kQgSets + set;
+      if (cols && r < rows) {
+        v[i] = qg_load<DT, VEC, true>(p, k0 + r, n0);
+      } else {
+#pragma unroll
+        for (auto& w : v[i].w) w = pk_u4v{0u, 0u, 0u, 0u};
+      }
+    }
+    QgMax<DT> m;
+    m.clear();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) m.take(v[i]);
+#pragma unroll
+    for (int i = 0; i < W; ++i) red[set][W * cl + i] = m.m[i];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kQgSets; ++u)
+#pragma unroll
+      for (int i = 0; i < W; ++i) m.take(i, red[u][W * cl + i]);
+    const QgScale q = qg_scale(p, m, mdt, g, n0, set == 0);
+    uint32_t redo = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int r = i * kQgSets + set;
+      if (cols && r < rows && qg_emit<DT, FAKE, false>(p, v[i], q, mdt, k0 + r, n0)) redo |= 1u << i;
+    }
+    for (; redo != 0; redo &= redo - 1) {
+      const int64_t k = k0 + (__builtin_ctz(redo) * kQgSets + set);
+      qg_emit<DT, FAKE, true>(p, qg_load<DT, VEC, false>(p, k, n0), q, mdt, k, n0);
+    }
+    __syncthreads();  // red is read before the next item writes it
+  }
+}
+
+constexpr int kQgLongThreads = 1024;
+constexpr int kQgLongSets = kQgLongThreads / 8;  // 64 columns per workgroup
+
+template <int DT, bool VEC, bool FAKE>
+__global__ __launch_bounds__(kQgLongThreads) void quantize_group_long_kernel(QgParams p) {
+  constexpr int W = QgMax<DT>::kWords;
+  __shared__ uint32_t red[kQgLongThreads / 64][8 * W];
+  const int t = threadIdx.x, set = t >> 3, lane = t & 63;
+  const int64_t tiles = cdiv(p.N, 64), items = tiles * cdiv(p.K, p.group);
+  const int mdt = p.half_math ? DT : PK_F32;
+  constexpr int U = 4;  // rows in flight per thread
+  for (int64_t b = blockIdx.x; b < items; b += gridDim.x) {
+    const int64_t g = b / tiles, n0 = (b - g * tiles) * 64 + 8 * (t & 7);
+    const int64_t k0 = g * p.group, k1 = min(k0 + p.group, p.K);
+    const bool cols = n0 < p.N;
+    QgMax<DT> m;
+    m.clear();
+    for (int64_t k = k0 + set; cols && k < k1; k += U * kQgLongSets) {
+      QgRow<DT> v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)  // past the group: the last row again
+        v[u] = qg_load<DT, VEC, false>(p, min(k + u * kQgLongSets, k1 - 1), n0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) m.take(v[u]);
+    }
+#pragma unroll
+    for (int i = 0; i < W; ++i) {
+      for (int x = 8; x < 64; x <<= 1) m.take(i, (uint32_t)__shfl_xor((int)m.m[i], x, 64));
+      if (lane < 8) red[t >> 6][W * lane + i] = m.m[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < W; ++i)
+      for (int u = 0; u < kQgLongThreads / 64; ++u) m.take(i, red[u][W * (t & 7) + i]);
+    const QgScale q = qg_scale(p, m, mdt, g, n0, set == 0);
+    for (int64_t k = k0 + set; cols && k < k1; k += U * kQgLongSets) {
+      QgRow<DT> v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        v[u] = qg_load<DT, VEC, false>(p, min(k + u * kQgLongSets, k1 - 1), n0);
+      uint32_t redo = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k + u * kQgLongSets < k1 &&
+            qg_emit<DT, FAKE, false>(p, v[u], q, mdt, k + u * kQgLongSets, n0))
+          redo |= 1u << u;
+      for (; redo != 0; redo &= redo - 1) {
+        const int64_t kr = k + __builtin_ctz(redo) * kQgLongSets;
+        qg_emit<DT, FAKE, true>(p, qg_load<DT, VEC, false>(p, kr, n0), q, mdt, kr, n0);
+      }
+    }
+    __syncthreads();  // red is read before the next item writes it
   }
 }
 
@@ -309,17 +555,29 @@ extern "C" int pk_quantize_group(const void* w, int w_dtype, int64_t K, int64_t 
   const int qmax = (1 << (bits - 1)) - 1;
   hipStream_t s = (hipStream_t)stream;
   const int64_t groups = cdiv(K, group);
-  if (qweight != nullptr || N % 8 == 0) {
-    int64_t items = cdiv(N, 8) * groups;
-    quantize_group_kernel<8><<<(unsigned)cdiv(items, kThreads), kThreads, 0, s>>>(
-        w, w_dtype, K, N, ldw, qmax, group, half_math, qweight, scales, scale_dtype, fake,
-        fake_dtype);
-  } else {
-    int64_t items = N * groups;
-    quantize_group_kernel<1><<<(unsigned)cdiv(items, kThreads), kThreads, 0, s>>>(
-        w, w_dtype, K, N, ldw, qmax, group, half_math, nullptr, scales, scale_dtype, fake,
-        fake_dtype);
-  }
+  const int es = w_dtype == PK_F32 ? 4 : 2;
+  const bool vec = N % 8 == 0 && (ldw * es) % 16 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+  const bool fake_vec = N % 8 == 0 && (reinterpret_cast<uintptr_t>(fake) & 15) == 0;
+  const QgParams p{w, K, N, ldw, qmax, group, half_math, qweight, scales, scale_dtype, fake,
+                   fake_dtype, fake_vec};
+  const bool longer = group > kQgRows;
+  const int64_t items = cdiv(N, longer ? 64 : 8 * kQgLanes) * groups;
+  const unsigned grid = (unsigned)(items < (1 << 20) ? items : (1 << 20));  // the kernels loop
+  auto go = [&](auto DT, auto V) {
+    constexpr int dt = decltype(DT)::value;
+    constexpr bool v = decltype(V)::value != 0;
+    if (longer && fake) quantize_group_long_kernel<dt, v, true><<<grid, kQgLongThreads, 0, s>>>(p);
+    else if (longer) quantize_group_long_kernel<dt, v, false><<<grid, kQgLongThreads, 0, s>>>(p);
+    else if (fake) quantize_group_kernel<dt, v, true><<<grid, kQgThreads, 0, s>>>(p);
+    else quantize_group_kernel<dt, v, false><<<grid, kQgThreads, 0, s>>>(p);
+  };
+  auto by_vec = [&](auto DT) {
+    if (vec) go(DT, pk_int_c<1>{});
+    else go(DT, pk_int_c<0>{});
+  };
+  if (w_dtype == PK_F32) by_vec(pk_int_c<PK_F32>{});
+  else if (w_dtype == PK_F16) by_vec(pk_int_c<PK_F16>{});
+  else by_vec(pk_int_c<PK_BF16>{});
   PK_LAUNCH_CHECK("pk_quantize_group");
   return PK_OK;
 }
