@@ -61,6 +61,22 @@ int pk_version(void);
 const char* pk_last_error(void);
 
 /* ------------------------------------------------------------------------------------- */
+/* Mailboxes                                                                             */
+/* ------------------------------------------------------------------------------------- */
+
+/* A mailbox is 64 bytes of pinned host memory, for one host thread at a time, into which a
+ * kernel posts a 32-bit value as message `seq` (a number the caller raises with every call
+ * that posts to it; 0 is never used). pk_mailbox_create returns NULL on failure.
+ * pk_mailbox_wait returns once message `seq` has come: the kernel that posts it has done its
+ * work, not what was launched after it. It polls for 0.3 ms and then synchronises `stream`
+ * (the stream of the posting call); PK_EHIP if the message has still not come. A mailbox may
+ * be destroyed once no call that posts to it is pending. No counterpart in the reference
+ * (torch's .item()). */
+void* pk_mailbox_create(void);
+void pk_mailbox_destroy(void* mailbox);
+int pk_mailbox_wait(const void* mailbox, uint32_t seq, uint32_t* value, void* stream);
+
+/* ------------------------------------------------------------------------------------- */
 /* Reductions and casts                                                                  */
 /* ------------------------------------------------------------------------------------- */
 
@@ -270,6 +286,15 @@ int pk_w4a16_launches(int M, int N, int K, int group_size, int split_k);
  * on the activation side. */
 int pk_w4a16_prep_activations(const void* x, int x_dtype, int64_t ldx, const float* in_scale,
                               float mul, void* y, int64_t ldy, int M, int K, void* stream);
+
+/* pk_w4a16_prep_activations that also answers whether a finite x became an infinite y (beyond
+ * fp16's 65504): posts 1 or 0 to `mailbox` as message `seq` (pk_mailbox_wait). `counter` is
+ * four bytes of device memory, zero before the call and left zero by it; calls ordered on one
+ * stream may share it. No counterpart in the reference, whose kernel takes bf16 as it is
+ * (gemm_int4.py:78). */
+int pk_w4a16_prep_checked(const void* x, int x_dtype, int64_t ldx, const float* in_scale, float mul,
+                          void* y, int64_t ldy, int M, int K, void* counter, void* mailbox,
+                          uint32_t seq, void* stream);
 
 /* Fixes the register-dequant kernel's (kernel id 3) layout for every later plan in the
  * process: 8 or 16 output columns per lane and 4 or 8 waves per workgroup; (0, 0) restores

@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import weakref
 from pathlib import Path
 
 import torch
@@ -36,9 +37,13 @@ _lib = None
 _lib_lock = threading.Lock()
 
 _vp, _i32, _i64, _f32, _sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_size_t
+_u32 = ctypes.c_uint32
 _SIGNATURES = {
     "pk_version": (_i32, []),
     "pk_last_error": (ctypes.c_char_p, []),
+    "pk_mailbox_create": (_vp, []),
+    "pk_mailbox_destroy": (None, [_vp]),
+    "pk_mailbox_wait": (_i32, [_vp, _u32, ctypes.POINTER(_u32), _vp]),
     "pk_absmax_workspace_bytes": (_sz, [_i64]),
     "pk_absmax": (_i32, [_vp, _i32, _i64, _vp, _vp, _sz, _vp]),
     "pk_quantize_int4": (_i32, [_vp, _i32, _i64, _f32, _vp, _vp]),
@@ -70,6 +75,8 @@ _SIGNATURES = {
     "pk_w4a16_strips_release": (None, [_vp]),
     "pk_w4a16_skinny_layout": (_i32, [_i32, _i32]),
     "pk_w4a16_prep_activations": (_i32, [_vp, _i32, _i64, _vp, _f32, _vp, _i64, _i32, _i32, _vp]),
+    "pk_w4a16_prep_checked": (_i32, [_vp, _i32, _i64, _vp, _f32, _vp, _i64, _i32, _i32, _vp, _vp,
+                                     _u32, _vp]),
     "pk_w4a16_gemm_noalloc": (_i32, [_vp, _i64, _vp, _i64, _vp, _i32, _f32, _vp, _i32, _i64, _i32, _i32,
                                      _i32, _i32, _vp]),
     "pk_w4a16_gemm_partials": (_i32, [_vp, _i64, _vp, _i64, _vp, _i32, _vp, _sz, _i32, _i32, _i32,
@@ -211,6 +218,53 @@ def workspace(device: torch.device, nbytes: int, stream: int | None = None) -> t
 
 
 # ---------------------------------------------------------------------------------------
+# Mailboxes: how a kernel hands the host one word without a stream synchronisation. One per
+# thread: a call that posts waits for its message before it returns, so a thread never has two
+# messages under way.
+# ---------------------------------------------------------------------------------------
+class _Mailbox(threading.local):
+    box: int | None = None
+    seq = 0
+
+    def next(self) -> tuple[int, int]:
+        """The thread's mailbox and the number of its next message."""
+        if self.box is None:
+            self.box = lib().pk_mailbox_create()
+            if not self.box:
+                self.box = None
+                raise PicoKernelsError("pk_mailbox_create failed: "
+                                       + lib().pk_last_error().decode(errors="replace"))
+            self.value = _u32(0)
+            # given back when the thread's locals go (every message has come by then)
+            self._guard = weakref.finalize(self.value, lib().pk_mailbox_destroy, self.box)
+            self._guard.atexit = False
+        self.seq = self.seq % 0xFFFFFFFF + 1
+        return self.box, self.seq
+
+    def wait(self, stream: int) -> int:
+        """The 32-bit value of the last message numbered here, posted on ``stream``."""
+        rc = lib().pk_mailbox_wait(self.box, self.seq, ctypes.byref(self.value), stream)
+        if rc != PK_OK:
+            _check(rc, "pk_mailbox_wait")
+        return self.value.value
+
+
+_mailbox = _Mailbox()
+
+# The arrival counter of the kernels that post, one line per (device, stream): zero-filled at
+# allocation, left zero by every call; calls on one stream are ordered.
+_post_counters: dict[tuple[int, int], torch.Tensor] = {}
+
+
+def _post_counter(device: torch.device, stream: int) -> int:
+    key = (device.index, stream)
+    t = _post_counters.get(key)
+    if t is None:
+        t = _post_counters[key] = torch.zeros(128, dtype=torch.uint8, device=device)
+    return t.data_ptr()
+
+
+# ---------------------------------------------------------------------------------------
 # Thin wrappers (one per C entry point). Inputs must already be on the GPU.
 # ---------------------------------------------------------------------------------------
 def absmax(x: torch.Tensor) -> torch.Tensor:
@@ -343,9 +397,51 @@ def check_fp16_range(x: torch.Tensor, what: str, converted: torch.Tensor | None 
         return
     bad = torch.isinf(converted) if converted is not None else x.abs() > FP16_MAX
     if bool((bad & torch.isfinite(x)).any()):
-        big = x[torch.isfinite(x)].abs().max().item()
-        raise ValueError(f"{what}: {x.dtype} activations up to |x| = {big:g} exceed fp16's range "
-                         f"(65504); the W4A16 kernels compute in fp16")
+        _raise_fp16_range(x, what)
+
+
+def _raise_fp16_range(x: torch.Tensor, what: str) -> None:
+    big = x[torch.isfinite(x)].abs().max().item()
+    raise ValueError(f"{what}: {x.dtype} activations up to |x| = {big:g} exceed fp16's range "
+                     f"(65504); the W4A16 kernels compute in fp16")
+
+
+class checked_activations:
+    """``w4a16_prep_activations`` with the range check of ``check_fp16_range`` in the same pass
+    (``pk_w4a16_prep_checked``): ``out`` is the fp16 tensor, for launches made inside the
+    ``with`` block; leaving the block waits for the check's answer and raises ``ValueError`` if
+    a finite element became infinite. Under graph capture (no host wait is possible) and for
+    inputs with nothing to check, the plain pass."""
+
+    def __init__(self, x: torch.Tensor, in_scale: torch.Tensor | None, mul: float, what: str):
+        self.x, self.what = x, what
+        self.stream = None
+        if (x.dtype == torch.float16 or not x.is_cuda or x.numel() == 0
+                or torch.cuda.is_current_stream_capturing()):
+            self.out = w4a16_prep_activations(x, in_scale, mul)
+            return
+        _gpu_args("w4a16_prep_activations", x, in_scale)
+        M, K = x.shape
+        if x.stride(1) != 1:
+            x = x.contiguous()
+        if in_scale is not None:
+            assert in_scale.dtype == torch.float32 and in_scale.is_contiguous() and in_scale.numel() == K
+        self.out = out = torch.empty((M, K), dtype=torch.float16, device=x.device)
+        stream = torch.cuda.current_stream(x.device).cuda_stream
+        counter = _post_counter(x.device, stream)
+        box, seq = _mailbox.next()
+        _check(lib().pk_w4a16_prep_checked(x.data_ptr(), pk_dtype(x.dtype), x.stride(0),
+                                           None if in_scale is None else in_scale.data_ptr(),
+                                           float(mul), out.data_ptr(), out.stride(0), M, K, counter,
+                                           box, seq, stream), "pk_w4a16_prep_checked")
+        self.stream = stream
+
+    def __enter__(self) -> torch.Tensor:
+        return self.out
+
+    def __exit__(self, *exc) -> None:
+        if self.stream is not None and _mailbox.wait(self.stream):
+            _raise_fp16_range(self.x, self.what)
 
 
 def _rows_ok(t: torch.Tensor) -> torch.Tensor:

@@ -52,6 +52,28 @@ bool splitk_in_l2_ok(hipStream_t stream);
 // has run, before that the XCC-count and environment rule alone.
 bool splitk_in_l2_possible();
 
+// A kernel's answer to the host (pk_mailbox_create / pk_mailbox_wait): `box` is a mailbox in
+// pinned host memory, `seq` the call's number. `counter` counts the launch's workgroups (zero
+// before the launch, left zero by it); null box: nothing is posted.
+struct Post {
+  uint64_t* box;
+  unsigned* counter;
+  uint32_t seq;
+};
+__device__ __forceinline__ void post(const Post& p, uint32_t value) {
+  __hip_atomic_store(p.box, ((uint64_t)p.seq << 32) | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+// One thread per workgroup, once: adds `add` (its low 16 bits 1) to the counter; true, with the
+// sum over all `total` (below 65536) workgroups, for the last to come. The workgroups run on
+// several XCDs: device-scope atomics, and nothing but the counter is handed over.
+__device__ __forceinline__ bool post_arrive(const Post& p, unsigned total, unsigned add, unsigned* sum) {
+  const unsigned old = __hip_atomic_fetch_add(p.counter, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if ((old & 0xffffu) != total - 1) return false;
+  __hip_atomic_store(p.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  *sum = old + add;
+  return true;
+}
+
 // Host: allow `kernel` up to `bytes` of dynamic LDS on the current device. The attribute is
 // set once per (device, kernel): `done` is a per-kernel bit set of the devices already done
 // (64 at most); concurrent first calls may both set it, which is harmless.

@@ -81,16 +81,20 @@ def int4_gemm(a: torch.Tensor, w_packed: torch.Tensor, scale: float,
     conversion is exact for 2^-17 <= |x| <= 65504 (and 0), so there the products with the
     exact integer codes, and the fp32 sums, are those of a bf16 dot; smaller magnitudes keep
     fp16's subnormal precision. A finite bf16 activation above 65504 raises ``ValueError``
-    (checked with one device reduction, except while a graph is being captured).
+    (checked in the same pass, except while a graph is being captured).
     """
     assert a.is_cuda and a.dtype in (torch.float16, torch.bfloat16)
     M, K = a.shape
     K2, N_half = w_packed.shape
     assert K2 == K, "int4_gemm: w_packed must be (K, N//2) for a of shape (M, K)"
     if a.dtype == torch.bfloat16:
-        _pk.check_fp16_range(a, "int4_gemm")
-        a = _pk.w4a16_prep_activations(a, None, 1.0)
-    N = N_half * 2
+        with _pk.checked_activations(a, None, 1.0, "int4_gemm") as a16:
+            return _int4_gemm_f16(a16, w_packed, scale)
+    return _int4_gemm_f16(a, w_packed, scale)
+
+
+def _int4_gemm_f16(a: torch.Tensor, w_packed: torch.Tensor, scale: float) -> torch.Tensor:
+    N = w_packed.shape[1] * 2
     assert N % 8 == 0, "int4_gemm: N must be a multiple of 8 (whole int32 words)"
     wp = w_packed if w_packed.is_cuda else w_packed.to(a.device)
     if not wp.is_contiguous():

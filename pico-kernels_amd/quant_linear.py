@@ -43,9 +43,9 @@ one copy. The copies are derived buffers, outside the state dict. ``codes()`` /
 
 The output has the input's dtype (fp16, bf16 or fp32, as ``nn.Linear``); other inputs are
 computed in fp16. A finite bf16 / fp32 activation whose fp16 form would be infinite (beyond
-65504, after the per-input scales for that scheme) raises ``ValueError``: one device reduction
-and synchronisation per call on such inputs, skipped under graph capture and when
-``QuantLinear.range_check`` is False (then such values become infinities, as torch's own fp16
+65504, after the per-input scales for that scheme) raises ``ValueError``: the cast's pass checks,
+and the call waits for its answer (not for the matmul behind it); skipped under graph capture
+and when ``QuantLinear.range_check`` is False (then such values become infinities, as torch's own fp16
 cast makes them). Weights need ``out % 8 == 0`` (whole int32 words) and ``in % 32 == 0``
 (the kernel's K), group layers ``in % group_size == 0``.
 """
@@ -274,26 +274,29 @@ class QuantLinear(nn.Module):
         # the bias is added in the matmul's epilogue (before the one rounding to out_dtype)
         if self.scheme == "per_input":
             # x * s / max s in fp16 (the input cast in the same pass), then max s in the epilogue
-            s = self.scales if self.scales.dtype == torch.float32 else self.scales.float()
-            xp = _pk.w4a16_prep_activations(x2, s, 1.0 / self._smax)
-            if self.range_check:
-                _pk.check_fp16_range(x2, "QuantLinear", xp)
-            if strips:
-                y = self._strips_call(out_dtype)(xp)
-            else:
-                y = _pk.w4a16_gemm(xp, self.qweight, None, 0, self._smax, out_dtype,
-                                   bias=self.bias, tiled=self.tiled)
+            s, mul = self.scales if self.scales.dtype == torch.float32 else self.scales.float(), 1.0 / self._smax
+        elif x2.dtype == torch.float16:
+            return self._matmul(x2, strips, out_dtype).reshape(*lead, self.out_features)
         else:
-            xp = x2 if x2.dtype == torch.float16 else _pk.w4a16_prep_activations(x2, None, 1.0)
-            if self.range_check and xp is not x2:
-                _pk.check_fp16_range(x2, "QuantLinear", xp)
-            if strips:
-                y = self._strips_call(out_dtype)(xp)
-            else:
-                s = self.scales if self.scales.dtype == torch.float16 else self.scales.half()
-                y = _pk.w4a16_gemm(xp, self.qweight, s, self.group_size, 1.0, out_dtype,
-                                   bias=self.bias, tiled=self.tiled)
+            s, mul = None, 1.0
+        if not self.range_check:
+            y = self._matmul(_pk.w4a16_prep_activations(x2, s, mul), strips, out_dtype)
+        else:
+            # the range check's answer is waited for once the matmul is launched as well
+            with _pk.checked_activations(x2, s, mul, "QuantLinear") as xp:
+                y = self._matmul(xp, strips, out_dtype)
         return y.reshape(*lead, self.out_features)
+
+    def _matmul(self, xp: torch.Tensor, strips: bool, out_dtype: torch.dtype) -> torch.Tensor:
+        """fp16 rows (prepared for the scheme) times the weight, plus the bias."""
+        if strips:
+            return self._strips_call(out_dtype)(xp)
+        if self.scheme == "per_input":
+            return _pk.w4a16_gemm(xp, self.qweight, None, 0, self._smax, out_dtype, bias=self.bias,
+                                  tiled=self.tiled)
+        s = self.scales if self.scales.dtype == torch.float16 else self.scales.half()
+        return _pk.w4a16_gemm(xp, self.qweight, s, self.group_size, 1.0, out_dtype, bias=self.bias,
+                              tiled=self.tiled)
 
     def _refresh(self) -> None:
         """Rebuild what derives from the buffers: the per-input epilogue scale and the decode
