@@ -72,6 +72,7 @@ const char* pk_last_error(void);
  * (the stream of the posting call); PK_EHIP if the message has still not come. A mailbox may
  * be destroyed once no call that posts to it is pending. No counterpart in the reference
  * (torch's .item()). */
+enum { PK_POST_COUNTER_BYTES = 2176 };
 void* pk_mailbox_create(void);
 void pk_mailbox_destroy(void* mailbox);
 int pk_mailbox_wait(const void* mailbox, uint32_t seq, uint32_t* value, void* stream);
@@ -86,6 +87,12 @@ int pk_mailbox_wait(const void* mailbox, uint32_t seq, uint32_t* value, void* st
 size_t pk_absmax_workspace_bytes(int64_t n);
 int pk_absmax(const void* x, int x_dtype, int64_t n, float* out_dev, void* workspace,
               size_t workspace_bytes, void* stream);
+
+/* pk_absmax in one launch that also posts the result (its fp32 bits) to `mailbox` as message
+ * `seq`. out_dev: 1 + pk_absmax_workspace_bytes(n) / 4 floats, the result first. `counters` as
+ * for pk_w4a16_prep_checked (they may be the same). */
+int pk_absmax_post(const void* x, int x_dtype, int64_t n, float* out_dev, void* counters,
+                   void* mailbox, uint32_t seq, void* stream);
 
 /* Per-tensor int4 codes: q[i] = int8(clamp(round(T(x[i] / scale)), -8, 7)) where T rounds
  * the fp32 quotient to x's dtype (fp16/bf16) exactly as a torch tensor op does, round is
@@ -130,6 +137,11 @@ int pk_quantize_group(const void* w, int w_dtype, int64_t K, int64_t N, int64_t 
  * Replaces `(x * scale).to(torch.float8_e4m3fn)` in gemm_fp8.quantize (gemm_fp8.py:95). */
 int pk_cast_e4m3(const void* x, int x_dtype, int64_t n, float scale, uint8_t* out,
                  void* stream);
+
+/* pk_cast_e4m3 with scale = 448 / absmax_dev[0] (the quotient in fp64, narrowed to fp32), for a
+ * maximum that is still being computed on the stream. */
+int pk_cast_e4m3_absmax(const void* x, int x_dtype, int64_t n, const float* absmax_dev,
+                        uint8_t* out, void* stream);
 
 /* ------------------------------------------------------------------------------------- */
 /* W4A16 matmul                                                                          */
@@ -288,12 +300,12 @@ int pk_w4a16_prep_activations(const void* x, int x_dtype, int64_t ldx, const flo
                               float mul, void* y, int64_t ldy, int M, int K, void* stream);
 
 /* pk_w4a16_prep_activations that also answers whether a finite x became an infinite y (beyond
- * fp16's 65504): posts 1 or 0 to `mailbox` as message `seq` (pk_mailbox_wait). `counter` is
- * four bytes of device memory, zero before the call and left zero by it; calls ordered on one
- * stream may share it. No counterpart in the reference, whose kernel takes bf16 as it is
+ * fp16's 65504): posts 1 or 0 to `mailbox` as message `seq` (pk_mailbox_wait). `counters`:
+ * PK_POST_COUNTER_BYTES of device memory, zero before the call and left zero by it; calls
+ * ordered on one stream may share them. No counterpart in the reference, whose kernel takes bf16 as it is
  * (gemm_int4.py:78). */
 int pk_w4a16_prep_checked(const void* x, int x_dtype, int64_t ldx, const float* in_scale, float mul,
-                          void* y, int64_t ldy, int M, int K, void* counter, void* mailbox,
+                          void* y, int64_t ldy, int M, int K, void* counters, void* mailbox,
                           uint32_t seq, void* stream);
 
 /* Fixes the register-dequant kernel's (kernel id 3) layout for every later plan in the

@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import struct
 import threading
 import weakref
 from pathlib import Path
@@ -46,12 +47,14 @@ _SIGNATURES = {
     "pk_mailbox_wait": (_i32, [_vp, _u32, ctypes.POINTER(_u32), _vp]),
     "pk_absmax_workspace_bytes": (_sz, [_i64]),
     "pk_absmax": (_i32, [_vp, _i32, _i64, _vp, _vp, _sz, _vp]),
+    "pk_absmax_post": (_i32, [_vp, _i32, _i64, _vp, _vp, _vp, _u32, _vp]),
     "pk_quantize_int4": (_i32, [_vp, _i32, _i64, _f32, _vp, _vp]),
     "pk_pack_int4": (_i32, [_vp, _i64, _i64, _i64, _vp, _vp]),
     "pk_unpack_int4": (_i32, [_vp, _i64, _i64, _vp, _vp]),
     "pk_quantize_group": (_i32, [_vp, _i32, _i64, _i64, _i64, _i32, _i32, _i32, _vp, _vp, _i32,
                                  _vp, _i32, _vp]),
     "pk_cast_e4m3": (_i32, [_vp, _i32, _i64, _f32, _vp, _vp]),
+    "pk_cast_e4m3_absmax": (_i32, [_vp, _i32, _i64, _vp, _vp, _vp]),
     "pk_w4a16_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32, _i32]),
     "pk_w4a16_launches": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "pk_w4a16_plan": (_i32, [_i32, _i32, _i32, _i32, _i32, ctypes.POINTER(_i32),
@@ -251,8 +254,10 @@ class _Mailbox(threading.local):
 
 _mailbox = _Mailbox()
 
-# The arrival counter of the kernels that post, one line per (device, stream): zero-filled at
-# allocation, left zero by every call; calls on one stream are ordered.
+POST_COUNTER_BYTES = 2176
+
+# The arrival counters of the kernels that post, per (device, stream): zero-filled at allocation,
+# left zero by every call; calls on one stream are ordered.
 _post_counters: dict[tuple[int, int], torch.Tensor] = {}
 
 
@@ -260,7 +265,7 @@ def _post_counter(device: torch.device, stream: int) -> int:
     key = (device.index, stream)
     t = _post_counters.get(key)
     if t is None:
-        t = _post_counters[key] = torch.zeros(128, dtype=torch.uint8, device=device)
+        t = _post_counters[key] = torch.zeros(POST_COUNTER_BYTES, dtype=torch.uint8, device=device)
     return t.data_ptr()
 
 
@@ -342,6 +347,30 @@ def cast_e4m3(x: torch.Tensor, scale: float) -> torch.Tensor:
     _check(lib().pk_cast_e4m3(x.data_ptr(), pk_dtype(x.dtype), x.numel(), float(scale),
                               out.data_ptr(), stream_of(x)), "pk_cast_e4m3")
     return out
+
+
+def absmax_cast_e4m3(x: torch.Tensor) -> tuple[torch.Tensor, float]:
+    """(e4m3(x * (448 / max|x|)), max|x|): the cast reads the maximum on the device, so it is
+    launched at once, and the host waits for the maximum alone."""
+    _gpu_args("cast_e4m3", x)
+    if torch.cuda.is_current_stream_capturing():
+        m = absmax(x).item()  # raises: no host wait while a graph is captured
+        return cast_e4m3(x, 448.0 / m), m
+    x = x.contiguous()
+    out = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
+    L = lib()
+    dt, n, stream = pk_dtype(x.dtype), x.numel(), stream_of(x)
+    m_dev = torch.empty(1 + L.pk_absmax_workspace_bytes(n) // 4, dtype=torch.float32, device=x.device)
+    counters = _post_counter(x.device, stream)
+    box, seq = _mailbox.next()
+    _check(L.pk_absmax_post(x.data_ptr(), dt, n, m_dev.data_ptr(), counters, box, seq, stream),
+           "pk_absmax_post")
+    try:
+        _check(L.pk_cast_e4m3_absmax(x.data_ptr(), dt, n, m_dev.data_ptr(), out.data_ptr(), stream),
+               "pk_cast_e4m3_absmax")
+    finally:
+        bits = _mailbox.wait(stream)
+    return out, struct.unpack("f", struct.pack("I", bits))[0]
 
 
 def w4a16_plan(M: int, N: int, K: int, group_size: int, split_k: int) -> tuple[int, int]:

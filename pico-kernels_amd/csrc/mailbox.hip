@@ -12,6 +12,8 @@
 
 using namespace pk;
 
+static_assert(kPostCounterBytes == PK_POST_COUNTER_BYTES, "header");
+
 extern "C" void* pk_mailbox_create(void) {
   void* box = nullptr;
   const hipError_t e = hipHostMalloc(&box, 64, hipHostMallocCoherent | hipHostMallocMapped | hipHostMallocPortable);

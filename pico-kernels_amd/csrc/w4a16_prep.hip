@@ -65,10 +65,8 @@ __global__ __launch_bounds__(kPrepThreads) void w4a16_prep_kernel(
     *reinterpret_cast<pk_half8*>(y + (int64_t)m * ldy + k0) = h;
   }
   if constexpr (CHECK) {
-    const int any = __syncthreads_or(bad);
-    unsigned sum;
-    if (threadIdx.x == 0 && post_arrive(pt, gridDim.x, any ? 0x10001u : 1u, &sum))
-      post(pt, sum > 0xffffu ? 1u : 0u);
+    bool any = __syncthreads_or(bad) != 0;
+    if (threadIdx.x == 0 && post_arrive(pt, &any)) post(pt, any ? 1u : 0u);
   }
 }
 
@@ -123,10 +121,10 @@ extern "C" int pk_w4a16_prep_activations(const void* x, int x_dtype, int64_t ldx
 }
 
 extern "C" int pk_w4a16_prep_checked(const void* x, int x_dtype, int64_t ldx, const float* in_scale,
-                                     float mul, void* y, int64_t ldy, int M, int K, void* counter,
+                                     float mul, void* y, int64_t ldy, int M, int K, void* counters,
                                      void* mailbox, uint32_t seq, void* stream) {
-  PK_REQUIRE(counter != nullptr && mailbox != nullptr, "pk_w4a16_prep_checked: null pointer");
+  PK_REQUIRE(counters != nullptr && mailbox != nullptr, "pk_w4a16_prep_checked: null pointer");
   return prep_launch("pk_w4a16_prep_checked", x, x_dtype, ldx, in_scale, mul, y, ldy, M, K,
-                     Post{static_cast<uint64_t*>(mailbox), static_cast<unsigned*>(counter), seq},
+                     Post{static_cast<uint64_t*>(mailbox), static_cast<unsigned*>(counters), seq},
                      (hipStream_t)stream);
 }

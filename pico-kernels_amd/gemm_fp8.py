@@ -30,8 +30,8 @@ def quantize(x: torch.Tensor) -> tuple[torch.Tensor, float]:
     Returns ``(x_fp8, scale)`` where ``x ~= x_fp8 / scale`` (gemm_fp8.py:89-95).
     """
     xg = _pk.to_gpu(x)
-    scale = _E4M3_MAX / _pk.absmax(xg).item()
-    x8 = _pk.cast_e4m3(xg, scale)
+    x8, absmax = _pk.absmax_cast_e4m3(xg)
+    scale = _E4M3_MAX / absmax
     return (x8 if x.is_cuda else x8.to(x.device)), scale
 
 
