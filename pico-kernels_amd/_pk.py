@@ -121,26 +121,40 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
-_strips_run_fast = None  # _pkcall.strips_run once probed, False when unavailable
+class _Calls:
+    """The library's functions by name, for the calls made once per layer and token: those the
+    CPython module ``_pkcall`` exposes (built beside the library by build.py: integers and floats
+    in, the status out, no ctypes conversion) when that module is there and the library was
+    loaded from its default path (the one ``_pkcall`` is linked against); else the ctypes
+    functions. Both make the same call."""
+
+    def __init__(self):
+        L = lib()
+        module = None
+        if LIB_PATH.resolve() == (HERE / LIB_NAME).resolve():
+            try:
+                import _pkcall as module
+            except ImportError:
+                pass
+        self.strips_run = getattr(module, "strips_run", L.pk_w4a16_strips_run)
+        for name in ("pk_w4a16_gemm", "pk_w4a16_gemm_bias", "pk_w4a16_gemm_tiled",
+                     "pk_w4a16_prep_checked", "pk_flash_decode"):
+            setattr(self, name, getattr(module, name, None) or getattr(L, name))
+
+
+_calls: _Calls | None = None
+
+
+def calls() -> _Calls:
+    global _calls
+    if _calls is None:
+        _calls = _Calls()
+    return _calls
 
 
 def strips_run_entry():
-    """``pk_w4a16_strips_run`` as the CPython module ``_pkcall`` exposes it (built beside the
-    library by build.py: six integers in, the status out, no ctypes conversion), when that
-    module is there and the library was loaded from its default path (the one ``_pkcall`` is
-    linked against); else the ctypes function. Both launch the same kernel."""
-    global _strips_run_fast
-    L = lib()
-    if _strips_run_fast is None:
-        _strips_run_fast = False
-        if LIB_PATH.resolve() == (HERE / LIB_NAME).resolve():
-            try:
-                import _pkcall
-
-                _strips_run_fast = _pkcall.strips_run
-            except ImportError:
-                pass
-    return _strips_run_fast or L.pk_w4a16_strips_run
+    """``pk_w4a16_strips_run``, through ``_pkcall`` where it can be."""
+    return calls().strips_run
 
 
 def _check(rc: int, what: str) -> None:
@@ -165,13 +179,18 @@ def _gpu_args(what: str, first: torch.Tensor, *others: torch.Tensor | None) -> N
     """Raise unless every tensor given (None skipped) lives on the GPU of ``first``: a host or
     other-device pointer handed to a kernel would fault the device instead of failing the call."""
     dev = first.get_device() if first.is_cuda else -1
-    if dev < 0 or any(t is not None and (not t.is_cuda or t.get_device() != dev) for t in others):
+    ok = dev >= 0
+    for t in others:
+        if t is not None and t.get_device() != dev:  # -1 on the host
+            ok = False
+    if not ok:
         raise ValueError(f"{what}: every tensor must be on one GPU (got "
                          + ", ".join(str(t.device) for t in (first, *others) if t is not None) + ")")
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The raw handle of the current stream of a GPU tensor's device."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def pk_dtype(dt: torch.dtype) -> int:
@@ -456,13 +475,15 @@ class checked_activations:
         if in_scale is not None:
             assert in_scale.dtype == torch.float32 and in_scale.is_contiguous() and in_scale.numel() == K
         self.out = out = torch.empty((M, K), dtype=torch.float16, device=x.device)
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        counter = _post_counter(x.device, stream)
+        stream = stream_of(x)
+        counters = _post_counter(x.device, stream)
         box, seq = _mailbox.next()
-        _check(lib().pk_w4a16_prep_checked(x.data_ptr(), pk_dtype(x.dtype), x.stride(0),
-                                           None if in_scale is None else in_scale.data_ptr(),
-                                           float(mul), out.data_ptr(), out.stride(0), M, K, counter,
-                                           box, seq, stream), "pk_w4a16_prep_checked")
+        rc = (_calls or calls()).pk_w4a16_prep_checked(
+            x.data_ptr(), pk_dtype(x.dtype), x.stride(0),
+            None if in_scale is None else in_scale.data_ptr(), float(mul), out.data_ptr(),
+            out.stride(0), M, K, counters, box, seq, stream)
+        if rc != PK_OK:
+            _check(rc, "pk_w4a16_prep_checked")
         self.stream = stream
 
     def __enter__(self) -> torch.Tensor:
@@ -712,18 +733,18 @@ def w4a16_gemm(a: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor | No
     split_k = int(split_k)
     key = (M, N, K, g, split_k)
     nbytes = _ws_bytes.get(key)
-    L = _lib if _lib is not None else lib()
     if nbytes is None:
-        nbytes = L.pk_w4a16_workspace_bytes(M, N, K, g, split_k)
+        nbytes = lib().pk_w4a16_workspace_bytes(M, N, K, g, split_k)
         if len(_ws_bytes) > 4096:
             _ws_bytes.clear()
         _ws_bytes[key] = nbytes
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    C = _calls or calls()
+    stream = stream_of(a)
     ws = workspace(dev, nbytes, stream) if nbytes else None
     if tiled:
         if not qweight.is_contiguous():
             raise ValueError("w4a16_gemm: block-layout weights must be contiguous")
-        rc = L.pk_w4a16_gemm_tiled(
+        rc = C.pk_w4a16_gemm_tiled(
             a.data_ptr(), a.stride(0), qweight.data_ptr(),
             None if scales is None else scales.data_ptr(), g, float(tensor_scale),
             None if bias is None else bias.data_ptr(),
@@ -734,7 +755,7 @@ def w4a16_gemm(a: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor | No
             _check(rc, "pk_w4a16_gemm_tiled")
         return out
     if bias is None:
-        rc = L.pk_w4a16_gemm(
+        rc = C.pk_w4a16_gemm(
             a.data_ptr(), a.stride(0), qweight.data_ptr(), qweight.stride(0),
             None if scales is None else scales.data_ptr(), g, float(tensor_scale), out.data_ptr(),
             _TORCH_TO_PK[out.dtype], out.stride(0), M, N, K, split_k,
@@ -742,7 +763,7 @@ def w4a16_gemm(a: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor | No
         if rc != PK_OK:
             _check(rc, "pk_w4a16_gemm")
         return out
-    rc = L.pk_w4a16_gemm_bias(
+    rc = C.pk_w4a16_gemm_bias(
         a.data_ptr(), a.stride(0), qweight.data_ptr(), qweight.stride(0),
         None if scales is None else scales.data_ptr(), g, float(tensor_scale), bias.data_ptr(),
         _TORCH_TO_PK[bias.dtype], out.data_ptr(), _TORCH_TO_PK[out.dtype], out.stride(0), M, N,
@@ -845,25 +866,40 @@ def flash_decode_launches(B: int, H: int, N: int, D: int, split: int) -> int:
     return int(lib().pk_flash_decode_launches(B, H, N, D, int(split)))
 
 
+# Workspace bytes per decode shape (a pure function of it).
+_fd_ws_bytes: dict[tuple[int, int, int, int, int], int] = {}
+
+
 def flash_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, split: int,
                  sm_scale: float) -> torch.Tensor:
     """(B, H, D) fp32 single-query attention of q (B, H, D) over k, v (B, H, N, D), all fp16
-    with unit stride along D (pk_flash_decode)."""
+    with unit stride along D (pk_flash_decode); (B, H, 1, D) for a 4-D q, its first row."""
     _gpu_args("flash_decode", q, k, v)
     B, H, N, D = k.shape
-
-    def _d_unit(t: torch.Tensor) -> torch.Tensor:
-        ok = t.stride(-1) == 1 and all(st % 8 == 0 for st in t.stride()[:-1]) and t.data_ptr() % 16 == 0
-        return t if ok else t.contiguous()
-
-    q, k, v = _d_unit(q), _d_unit(k), _d_unit(v)
-    out = torch.empty((B, H, D), dtype=torch.float32, device=q.device)
-    nbytes = lib().pk_flash_decode_workspace_bytes(B, H, N, D, int(split))
-    ws = workspace(q.device, nbytes)  # zero-filled counters, shared with the GEMMs
-    _check(lib().pk_flash_decode(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0),
-                                 k.stride(1), k.stride(2), v.data_ptr(), v.stride(0), v.stride(1),
-                                 v.stride(2), B, H, N, D, int(split), float(sm_scale),
-                                 out.data_ptr(), 0 if ws is None else ws.data_ptr(),
-                                 0 if ws is None else ws.numel(), stream_of(q)),
-           "pk_flash_decode")
+    sq, sk, sv = q.stride(), k.stride(), v.stride()
+    if sq[-1] != 1 or (sq[0] | sq[1]) & 7 or q.data_ptr() & 15:
+        q = q.contiguous()
+        sq = q.stride()
+    if sk[3] != 1 or (sk[0] | sk[1] | sk[2]) & 7 or k.data_ptr() & 15:
+        k = k.contiguous()
+        sk = k.stride()
+    if sv[3] != 1 or (sv[0] | sv[1] | sv[2]) & 7 or v.data_ptr() & 15:
+        v = v.contiguous()
+        sv = v.stride()
+    out = q.new_empty((B, H, D) if len(sq) == 3 else (B, H, 1, D), dtype=torch.float32)
+    split = int(split)
+    key = (B, H, N, D, split)
+    nbytes = _fd_ws_bytes.get(key)
+    if nbytes is None:
+        if len(_fd_ws_bytes) > 4096:
+            _fd_ws_bytes.clear()
+        nbytes = _fd_ws_bytes[key] = lib().pk_flash_decode_workspace_bytes(B, H, N, D, split)
+    stream = stream_of(q)
+    ws = workspace(q.device, nbytes, stream)  # zero-filled counters, shared with the GEMMs
+    rc = (_calls or calls()).pk_flash_decode(
+        q.data_ptr(), sq[0], sq[1], k.data_ptr(), sk[0], sk[1], sk[2], v.data_ptr(), sv[0], sv[1],
+        sv[2], B, H, N, D, split, float(sm_scale), out.data_ptr(),
+        0 if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), stream)
+    if rc != PK_OK:
+        _check(rc, "pk_flash_decode")
     return out

@@ -81,7 +81,7 @@ def _link(objs: list[Path], out: Path, verbose: bool) -> None:
 
 
 def _build_pkcall(lib: Path, verbose: bool) -> Path:
-    """The CPython module ``_pkcall`` (csrc/pkcall.c: the prepared decode call without ctypes),
+    """The CPython module ``_pkcall`` (csrc/pkcall.c: the calls made once per layer, without ctypes),
     linked against ``lib`` by path (rpath $ORIGIN)."""
     import sysconfig
 

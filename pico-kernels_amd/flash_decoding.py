@@ -48,13 +48,14 @@ class KVCache:
 
 def flash_decoding(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                    split_size: int = 256) -> torch.Tensor:
-    B, H, _, D = q.shape
+    _, _, rows, D = q.shape
     N = k.shape[2]
+    if rows < 1:
+        raise IndexError("flash_decoding: q has no row")
     assert N % split_size == 0, "N must divide split_size"
     assert q.is_cuda and k.is_cuda and v.is_cuda, "flash_decoding: inputs must be on the GPU"
     assert q.dtype == k.dtype == v.dtype == torch.float16, "flash_decoding: fp16 q, k, v expected"
-    o = _pk.flash_decode(q[:, :, 0, :], k, v, split_size, 1.0 / math.sqrt(D))
-    return o[:, :, None, :]
+    return _pk.flash_decode(q, k, v, split_size, 1.0 / math.sqrt(D))
 
 
 def eager_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:

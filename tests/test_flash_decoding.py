@@ -186,3 +186,19 @@ def test_graph_replays(cuda):
         torch.cuda.synchronize(cuda)
         assert torch.equal(out, eager), rep
         assert torch.equal(_pk.flash_decode(qg, kg, vg, split, scale), eager)
+
+
+@pytest.mark.gpu
+def test_query_forms(cuda):
+    """A strided q (a row of a longer one, read in place), a q that has to be copied, and no row."""
+    from flash_decoding import flash_decoding
+
+    g = torch.Generator(device="cuda").manual_seed(5)
+    wide = torch.randn(2, 4, 3, 72, device=cuda, dtype=torch.float16, generator=g)
+    k, v = (torch.randn(2, 4, 512, 64, device=cuda, dtype=torch.float16, generator=g) for _ in range(2))
+    for q in (wide[:, :, 1:2, :64], wide[:, :, 1:2, 3:67], wide[:, :, 1:3, :64]):
+        o = flash_decoding(q, k, v)
+        assert o.shape == (2, 4, 1, 64) and o.is_contiguous()
+        assert torch.equal(o, flash_decoding(q[:, :, :1].contiguous(), k, v))
+    with pytest.raises(IndexError):
+        flash_decoding(wide[:, :, :0, :64], k, v)
