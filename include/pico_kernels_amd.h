@@ -225,6 +225,13 @@ int pk_w4a16_gemm_strips(const void* a, int64_t lda, const uint8_t* qstrips, con
                          int group_size, float tensor_scale, const void* bias, int bias_dtype,
                          void* c, int c_dtype, int64_t ldc, int M, int N, int K, void* stream);
 
+/* pk_w4a16_gemm_strips for 5 <= M <= 64 rows: the same weights, arguments and conditions, one
+ * launch with no split-K partials, a fixed summation order (bitwise reproducible). Replaces
+ * gemm_int4.int4_gemm (gemm_int4.py:75-92) for a batch of rows on the strip layout. */
+int pk_w4a16_gemm_strips_rows(const void* a, int64_t lda, const uint8_t* qstrips, const void* sstrips,
+                              int group_size, float tensor_scale, const void* bias, int bias_dtype,
+                              void* c, int c_dtype, int64_t ldc, int M, int N, int K, void* stream);
+
 /* Fix the strip GEMV's 1 KB blocks per wave (2, 4 or 8) for later calls, or 0 for the
  * automatic choice; for measurements. No counterpart in the reference. */
 int pk_w4a16_strips_config(int blocks_per_wave);
@@ -251,6 +258,8 @@ void* pk_w4a16_strips_prepare(const uint8_t* qstrips, const void* sstrips, int g
                               float tensor_scale, const void* bias, int bias_dtype, int c_dtype,
                               int N, int K, int64_t lda);
 int pk_w4a16_strips_run(void* prepared, const void* a, void* c, int64_t ldc, int M, void* stream);
+/* pk_w4a16_gemm_strips_rows (5 <= M <= 64) by a prepared handle. */
+int pk_w4a16_strips_run_rows(void* prepared, const void* a, void* c, int64_t ldc, int M, void* stream);
 void pk_w4a16_strips_release(void* prepared);
 
 /* pk_w4a16_strips_run with timing: the dispatch itself records start_event (a hipEvent_t) as

@@ -69,11 +69,14 @@ _SIGNATURES = {
     "pk_w4a16_tiled_rows_per_call": (_i64, [_i64, _i64]),
     "pk_w4a16_gemm_strips": (_i32, [_vp, _i64, _vp, _vp, _i32, _f32, _vp, _i32, _vp, _i32, _i64,
                                     _i32, _i32, _i32, _vp]),
+    "pk_w4a16_gemm_strips_rows": (_i32, [_vp, _i64, _vp, _vp, _i32, _f32, _vp, _i32, _vp, _i32, _i64,
+                                         _i32, _i32, _i32, _vp]),
     "pk_w4a16_strips_config": (_i32, [_i32]),
     "pk_w4a16_strips_plan": (_i32, [_i32, _i32, _i32, ctypes.POINTER(_i32), ctypes.POINTER(_i32),
                                     ctypes.POINTER(_i32)]),
     "pk_w4a16_strips_prepare": (_vp, [_vp, _vp, _i32, _f32, _vp, _i32, _i32, _i32, _i32, _i64]),
     "pk_w4a16_strips_run": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
+    "pk_w4a16_strips_run_rows": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp]),
     "pk_w4a16_strips_run_events": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp]),
     "pk_w4a16_strips_release": (None, [_vp]),
     "pk_w4a16_skinny_layout": (_i32, [_i32, _i32]),
@@ -138,6 +141,7 @@ class _Calls:
                 pass
         self.strips_run = getattr(module, "strips_run", L.pk_w4a16_strips_run)
         for name in ("pk_w4a16_gemm", "pk_w4a16_gemm_bias", "pk_w4a16_gemm_tiled",
+                     "pk_w4a16_gemm_strips", "pk_w4a16_gemm_strips_rows", "pk_w4a16_strips_run_rows",
                      "pk_w4a16_prep_checked", "pk_flash_decode"):
             setattr(self, name, getattr(module, name, None) or getattr(L, name))
 
@@ -583,9 +587,10 @@ def unstrip_scales(sstrips: torch.Tensor) -> torch.Tensor:
 def w4a16_gemm_strips(a: torch.Tensor, qstrips: torch.Tensor, sstrips: torch.Tensor | None,
                       group_size: int, tensor_scale: float, out_dtype: torch.dtype,
                       out: torch.Tensor | None = None,
-                      bias: torch.Tensor | None = None) -> torch.Tensor:
+                      bias: torch.Tensor | None = None, rows: bool = False) -> torch.Tensor:
     """out = tensor_scale * (a @ dequant(q, s)) (+ bias) for 1..8 rows of fp16 activations on
-    strip-layout codes and scales (strip_weights / strip_scales; pk_w4a16_gemm_strips)."""
+    strip-layout codes and scales (strip_weights / strip_scales; pk_w4a16_gemm_strips), or 5..64
+    with ``rows`` (pk_w4a16_gemm_strips_rows)."""
     _gpu_args("w4a16_gemm_strips", a, qstrips, sstrips, out, bias)
     M, K = a.shape
     N = qstrips.shape[1] * 8
@@ -593,28 +598,37 @@ def w4a16_gemm_strips(a: torch.Tensor, qstrips: torch.Tensor, sstrips: torch.Ten
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     g = int(group_size) if sstrips is not None else 0
-    L = _lib if _lib is not None else lib()
-    rc = L.pk_w4a16_gemm_strips(
+    C = _calls or calls()
+    rc = (C.pk_w4a16_gemm_strips_rows if rows else C.pk_w4a16_gemm_strips)(
         a.data_ptr(), a.stride(0), qstrips.data_ptr(),
         None if sstrips is None else sstrips.data_ptr(), g, float(tensor_scale),
         None if bias is None else bias.data_ptr(),
         _TORCH_TO_PK[bias.dtype] if bias is not None else PK_F16, out.data_ptr(),
-        _TORCH_TO_PK[out.dtype], out.stride(0), M, N, K,
-        torch.cuda.current_stream(a.device).cuda_stream)
+        _TORCH_TO_PK[out.dtype], out.stride(0), M, N, K, stream_of(a))
     if rc != PK_OK:
         _check(rc, "pk_w4a16_gemm_strips")
     return out
 
 
+def strip_rows_from(N: int) -> int:
+    """Rows from which a strip-layout call of N columns runs the batch kernel
+    (pk_w4a16_strips_run_rows) instead of the decode kernel: 9, or 5 where two or four strips
+    share a workgroup (more than 256 strips). Measured on MI355X at M = 8, decode / batch kernel:
+    4096 x 4096 5.8 / 5.7 us, 14336 x 4096 11.8 / 12.9; 4096 x 6144 7.5 / 6.5, 4096 x 14336
+    11.5 / 10.1, 8192 x 14336 20.0 / 15.4."""
+    return 5 if N > 16 * 256 else 9
+
+
 class PreparedStrips:
-    """``pk_w4a16_gemm_strips`` bound to one strip-layout weight copy through
+    """``pk_w4a16_gemm_strips`` (1..8 rows) and ``pk_w4a16_gemm_strips_rows`` (5..64) bound to one strip-layout weight copy through
     ``pk_w4a16_strips_prepare``: the fixed arguments are checked and the launches for 1..8 rows
     planned once, so a call passes only the activations, the output, the row count and the
     stream (what an eager decode loop pays per layer). Activations must be 16-byte aligned with
     row stride ``lda`` (elements; default K). The tensors stay referenced here, and must stay
     in place, while the object lives (QuantLinear drops it when its buffers move or change)."""
 
-    __slots__ = ("h", "N", "K", "lda", "out_dtype", "dev", "run", "run_events", "release", "_keep")
+    __slots__ = ("h", "N", "K", "lda", "out_dtype", "dev", "run", "run_rows", "rows_from",
+                 "run_events", "release", "_keep")
 
     def __init__(self, qstrips: torch.Tensor, sstrips: torch.Tensor | None, group_size: int,
                  tensor_scale: float, out_dtype: torch.dtype, bias: torch.Tensor | None = None,
@@ -636,6 +650,7 @@ class PreparedStrips:
             raise PicoKernelsError("pk_w4a16_strips_prepare failed: "
                                    + L.pk_last_error().decode(errors="replace"))
         self.run, self.release = strips_run_entry(), L.pk_w4a16_strips_release
+        self.run_rows, self.rows_from = calls().pk_w4a16_strips_run_rows, strip_rows_from(self.N)
         self.run_events = L.pk_w4a16_strips_run_events
 
     def __del__(self):
@@ -662,8 +677,9 @@ class PreparedStrips:
               or out.get_device() != self.dev):
             raise ValueError(f"PreparedStrips: out must be ({M}, {self.N}) {self.out_dtype} with "
                              f"unit column stride on cuda:{self.dev}")
-        rc = self.run(self.h, a.data_ptr(), out.data_ptr(), out.stride(0), M,
-                      torch._C._cuda_getCurrentRawStream(self.dev))
+        run = self.run if M < self.rows_from else self.run_rows
+        rc = run(self.h, a.data_ptr(), out.data_ptr(), out.stride(0), M,
+                 torch._C._cuda_getCurrentRawStream(self.dev))
         if rc != PK_OK:
             _check(rc, "pk_w4a16_strips_run")
         return out

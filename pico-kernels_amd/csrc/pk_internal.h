@@ -125,6 +125,11 @@ int strips_launch(const void* a, int64_t lda, const uint8_t* qs, const void* ss,
                   OutEpi epi, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
                   hipStream_t stream);
 bool strips_config_set(int blocks_per_wave);
+// The same weights at 5 <= M <= 64 (w4a16_strip_rows.hip).
+constexpr int kStripRowsMinM = 5, kStripRowsMaxM = 64;
+int strip_rows_launch(const void* a, int64_t lda, const uint8_t* qs, const void* ss, int group,
+                      OutEpi epi, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
+                      hipStream_t stream);
 
 // W4A16 for kSkinnyMinM <= M <= kSkinnyMaxM (w4a16_skinny.hip): weights to registers, MFMA
 // per 16 activation rows, LDS reduction over the workgroup's waves, split-K partials.

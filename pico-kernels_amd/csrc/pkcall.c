@@ -105,6 +105,11 @@ PKCALL(pk_w4a16_gemm_tiled, "plppi" "fpipil" "iiii" "plp",
        pk_w4a16_gemm_tiled(a[0].p, a[1].l, a[2].p, a[3].p, a[4].i, a[5].f, a[6].p, a[7].i, a[8].p,
                            a[9].i, a[10].l, a[11].i, a[12].i, a[13].i, a[14].i, a[15].p,
                            (size_t)a[16].l, a[17].p))
+PKCALL(pk_w4a16_strips_run_rows, "pppl" "ip",
+       pk_w4a16_strips_run_rows(a[0].p, a[1].p, a[2].p, a[3].l, a[4].i, a[5].p))
+PKCALL(pk_w4a16_gemm_strips_rows, "plpp" "ifpi" "pil" "iiip",
+       pk_w4a16_gemm_strips_rows(a[0].p, a[1].l, a[2].p, a[3].p, a[4].i, a[5].f, a[6].p, a[7].i,
+                                 a[8].p, a[9].i, a[10].l, a[11].i, a[12].i, a[13].i, a[14].p))
 PKCALL(pk_w4a16_prep_checked, "pilpf" "plii" "ppup",
        pk_w4a16_prep_checked(a[0].p, a[1].i, a[2].l, a[3].p, a[4].f, a[5].p, a[6].l, a[7].i, a[8].i,
                              a[9].p, a[10].p, a[11].u, a[12].p))
@@ -119,7 +124,7 @@ static PyMethodDef pkcall_methods[] = {
     {"strips_run", (PyCFunction)(void (*)(void))pkcall_strips_run, METH_FASTCALL,
      "pk_w4a16_strips_run(handle, a, c, ldc, M, stream) -> status"},
     ENTRY(pk_w4a16_gemm), ENTRY(pk_w4a16_gemm_bias), ENTRY(pk_w4a16_gemm_tiled),
-    ENTRY(pk_w4a16_prep_checked), ENTRY(pk_flash_decode),
+    ENTRY(pk_w4a16_strips_run_rows), ENTRY(pk_w4a16_gemm_strips_rows), ENTRY(pk_w4a16_prep_checked), ENTRY(pk_flash_decode),
     {NULL, NULL, 0, NULL},
 };
 

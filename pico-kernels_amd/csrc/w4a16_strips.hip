@@ -539,19 +539,21 @@ extern "C" int pk_w4a16_strips_plan(int M, int N, int K, int* strips_per_workgro
 namespace {
 int check_strips(const char* name, const void* a, int64_t lda, const uint8_t* qstrips,
                  const void* sstrips, int group_size, const void* bias, int bias_dtype,
-                 const void* c, int c_dtype, int64_t ldc, int M, int N, int K) {
+                 const void* c, int c_dtype, int64_t ldc, int M, int N, int K,
+                 int min_m = 1, int max_m = 8) {
   auto al = [](const void* q, unsigned b) { return (reinterpret_cast<uintptr_t>(q) & (b - 1)) == 0; };
   PK_REQUIRE(qstrips != nullptr, "%s: null weights", name);
-  PK_REQUIRE(M >= 1 && M <= 8, "%s: M=%d (the strip layout serves 1..8 rows)", name, M);
+  PK_REQUIRE(M >= min_m && M <= max_m, "%s: M=%d (the strip layout serves %d..%d rows)", name, M,
+             min_m, max_m);
   PK_REQUIRE(N >= 16 && N % 16 == 0 && K >= 128 && K % 128 == 0,
              "%s: needs N %% 16 == 0 and K %% 128 == 0 (N=%d K=%d)", name, N, K);
-  PK_REQUIRE(sstrips == nullptr || strips_shape_ok(M, N, K, group_size, true),
+  PK_REQUIRE(sstrips == nullptr || strips_shape_ok(M < 8 ? M : 8, N, K, group_size, true),
              "%s: group_size=%d must be a multiple of 32 dividing K=%d and either divide 128 or "
              "be a multiple of it", name, group_size, K);
   PK_REQUIRE(a == nullptr || (lda >= K && lda % 8 == 0 && al(a, 16)),
              "%s: A rows must be 16-byte aligned", name);
   PK_REQUIRE((int64_t)M * lda * 2 < (1ll << 31), "%s: A beyond 2 GiB", name);
-  PK_REQUIRE((int64_t)K * 8 < (1ll << 31), "%s: K=%d too large", name, K);
+  PK_REQUIRE((int64_t)K * (max_m > 8 ? 32 : 8) < (1ll << 31), "%s: K=%d too large", name, K);
   PK_REQUIRE(al(qstrips, 16) && (sstrips == nullptr || al(sstrips, 8)),
              "%s: weights must be 16-byte and scales 8-byte aligned", name);
   PK_REQUIRE(c == nullptr || ldc >= N, "%s: ldc < N", name);
@@ -566,8 +568,11 @@ int check_strips(const char* name, const void* a, int64_t lda, const uint8_t* qs
 // only afterwards, so concurrent runs on different streams may share it).
 struct StripsPrepared {
   StripPlan plan[8];  // by M - 1
-  int N;
+  int N, K, group, c_dtype;
   int64_t lda;
+  const uint8_t* qs;
+  const void* ss;
+  OutEpi epi;
 };
 }  // namespace
 
@@ -583,6 +588,19 @@ extern "C" int pk_w4a16_gemm_strips(const void* a, int64_t lda, const uint8_t* q
                        c, c_dtype, ldc, M, N, K, (hipStream_t)stream);
 }
 
+extern "C" int pk_w4a16_gemm_strips_rows(const void* a, int64_t lda, const uint8_t* qstrips,
+                                         const void* sstrips, int group_size, float tensor_scale,
+                                         const void* bias, int bias_dtype, void* c, int c_dtype,
+                                         int64_t ldc, int M, int N, int K, void* stream) {
+  PK_REQUIRE(a != nullptr && c != nullptr, "pk_w4a16_gemm_strips_rows: null pointer");
+  const int rc = check_strips("pk_w4a16_gemm_strips_rows", a, lda, qstrips, sstrips, group_size,
+                              bias, bias_dtype, c, c_dtype, ldc, M, N, K, kStripRowsMinM, kStripRowsMaxM);
+  if (rc != PK_OK) return rc;
+  return strip_rows_launch(a, lda, qstrips, sstrips, group_size,
+                           OutEpi(tensor_scale, bias, bias_dtype), c, c_dtype, ldc, M, N, K,
+                           (hipStream_t)stream);
+}
+
 extern "C" void* pk_w4a16_strips_prepare(const uint8_t* qstrips, const void* sstrips,
                                          int group_size, float tensor_scale, const void* bias,
                                          int bias_dtype, int c_dtype, int N, int K, int64_t lda) {
@@ -595,7 +613,13 @@ extern "C" void* pk_w4a16_strips_prepare(const uint8_t* qstrips, const void* sst
     return nullptr;
   }
   h->N = N;
+  h->K = K;
+  h->group = group_size;
+  h->c_dtype = c_dtype;
   h->lda = lda;
+  h->qs = qstrips;
+  h->ss = sstrips;
+  h->epi = OutEpi(tensor_scale, bias, bias_dtype);
   for (int m = 1; m <= 8; ++m)
     strips_plan(qstrips, sstrips, group_size, OutEpi(tensor_scale, bias, bias_dtype), c_dtype, m,
                 N, K, lda, &h->plan[m - 1]);
@@ -619,6 +643,19 @@ int strips_run_checked(const char* name, void* prepared, const void* a, void* c,
 extern "C" int pk_w4a16_strips_run(void* prepared, const void* a, void* c, int64_t ldc, int M,
                                    void* stream) {
   return strips_run_checked("pk_w4a16_strips_run", prepared, a, c, ldc, M, stream, nullptr, nullptr);
+}
+
+extern "C" int pk_w4a16_strips_run_rows(void* prepared, const void* a, void* c, int64_t ldc, int M,
+                                        void* stream) {
+  const char* name = "pk_w4a16_strips_run_rows";
+  auto* h = static_cast<StripsPrepared*>(prepared);
+  PK_REQUIRE(h != nullptr && a != nullptr && c != nullptr, "%s: null pointer", name);
+  const int rc = check_strips(name, a, h->lda, h->qs, h->ss, h->group, h->epi.bias,
+                              h->epi.bias_dtype, c, h->c_dtype, ldc, M, h->N, h->K, kStripRowsMinM,
+                              kStripRowsMaxM);
+  if (rc != PK_OK) return rc;
+  return strip_rows_launch(a, h->lda, h->qs, h->ss, h->group, h->epi, c, h->c_dtype, ldc, M, h->N,
+                           h->K, (hipStream_t)stream);
 }
 
 extern "C" int pk_w4a16_strips_run_events(void* prepared, const void* a, void* c, int64_t ldc,

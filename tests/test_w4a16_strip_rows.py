@@ -1,0 +1,102 @@
+"""The strip layout's batch kernel (pk_w4a16_gemm_strips_rows): every number of strips per workgroup
+(with a last workgroup that has fewer), 128-row blocks that do not divide among the waves, 16-row
+activation blocks with a remainder, every kind of group, bias and output dtype, strided
+activations; and QuantLinear's rule for it."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import _pk
+import gemm_int4
+import oracle
+import quant_linear
+
+SHAPES = [(128, 16), (384, 48), (1152, 4096 + 16), (1024, 8192 + 48), (2176, 16400)]
+
+
+def _layer(K, N, group, seed):
+    g = torch.Generator().manual_seed(seed)
+    w = (torch.randn(K, N, generator=g) * 0.02).half()
+    codes, _, s16 = oracle.rtn_group_codes(w.numpy(), 4, group or K)
+    return codes, s16 if group else None
+
+
+def _want(a, codes, s16, group, scale, bias):
+    """fp64 product of the same codes and scales."""
+    w = torch.from_numpy(codes).double()
+    if s16 is not None:
+        w = w * torch.from_numpy(s16.astype(np.float64)).repeat_interleave(group, 0)
+    y = scale * (a.double() @ w.to(a.device))
+    return y if bias is None else y + bias.double()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,N", SHAPES)
+@pytest.mark.parametrize("group", [128, 64, 32, 0, -1])
+def test_against_fp64(cuda, K, N, group):
+    group = K if group < 0 else group  # -1: one group over all of K
+    codes, s16 = _layer(K, N, group, K + N)
+    qw = torch.from_numpy(oracle.pack_int4_n(codes)).to(cuda).view(torch.int32)
+    qs = _pk.strip_weights(qw)
+    ss = None if s16 is None else _pk.strip_scales(torch.from_numpy(s16).to(cuda))
+    g = torch.Generator(device=cuda).manual_seed(N)
+    bias = torch.randn(N, generator=g, device=cuda)
+    for M in (5, 16, 17, 32, 33, 64):
+        a = torch.randn(M, K + 8, generator=g, device=cuda).half()[:, :K]
+        want = _want(a, codes, s16, group, 0.5, bias)
+        y = _pk.w4a16_gemm_strips(a, qs, ss, group, 0.5, torch.float32, bias=bias, rows=True)
+        # exact products, fp32 sums of K of them in blocks of 128: K / 128 + 128 roundings of
+        # 2^-24 on sums of the size of the result bound the 2-norm error far below 2e-5
+        assert (y - want).norm() <= 2e-5 * want.norm(), (M, group)
+        assert torch.equal(y, _pk.w4a16_gemm_strips(a, qs, ss, group, 0.5, torch.float32, bias=bias, rows=True))
+        for dt in (torch.float16, torch.bfloat16):  # one rounding of the same fp32 sums
+            z = _pk.w4a16_gemm_strips(a, qs, ss, group, 0.5, dt, bias=bias, rows=True)
+            assert torch.equal(z, y.to(dt))
+
+
+@pytest.mark.gpu
+def test_prepared_call_and_limits(cuda):
+    codes, s16 = _layer(512, 4352, 128, 1)
+    qw = torch.from_numpy(oracle.pack_int4_n(codes)).to(cuda).view(torch.int32)
+    qs, ss = _pk.strip_weights(qw), _pk.strip_scales(torch.from_numpy(s16).to(cuda))
+    call = _pk.PreparedStrips(qs, ss, 128, 1.0, torch.float16)
+    assert call.rows_from == 5 and _pk.strip_rows_from(4096) == 9
+    for M in (5, 9, 64):
+        a = torch.randn(M, 512, device=cuda).half()
+        assert torch.equal(call(a), _pk.w4a16_gemm_strips(a, qs, ss, 128, 1.0, torch.float16, rows=True))
+    for M in (0, 65):
+        with pytest.raises(_pk.PicoKernelsError):
+            call(torch.zeros(M, 512, device=cuda, dtype=torch.float16))
+    with pytest.raises(_pk.PicoKernelsError):
+        _pk.w4a16_gemm_strips(torch.zeros(4, 512, device=cuda, dtype=torch.float16), qs, ss, 128, 1.0,
+                              torch.float16, rows=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scheme", ["group", "per_input"])
+@pytest.mark.parametrize("out_f", [1024, 4112])
+def test_quant_linear_batches(cuda, scheme, out_f):
+    """QuantLinear agrees with itself without the strip copy at every row count around the rule's
+    ends, for fp16 and bf16 inputs and a 3-D input."""
+    lin = torch.nn.Linear(1280, out_f, device=cuda, dtype=torch.float16)
+    q = quant_linear.QuantLinear.from_linear(lin, 128, None if scheme == "group" else "rtn")
+    assert q.decode
+    first, last = quant_linear.strip_rows(1280, out_f, q.tiled)
+    for M in (1, 4, 5, 8, 9, 16, 33, last, last + 1):
+        for dt in (torch.float16, torch.bfloat16):
+            x = torch.randn(M, 1280, device=cuda).to(dt)
+            y = q(x)
+            ref = x.double() @ q.dequantized_weight().double().t() + q.bias.double()
+            assert (y.double() - ref).norm() <= (1e-3 if dt == torch.float16 else 6e-3) * ref.norm()
+            if M == 16:
+                assert torch.equal(q(x.view(2, 8, -1)).view(M, -1), y)
+
+
+def test_rule():
+    r = quant_linear.strip_rows
+    assert r(4096, 8192, True) == (9, 64) and r(4096, 8208, True) == (9, 32)
+    assert r(8192, 4096, True) == (9, 32) and r(8320, 4096, True) == (9, 16)
+    assert r(14336, 28672, False) == (5, 64)
