@@ -571,12 +571,14 @@ def bench_llama_sweep(dev, iters: int = 50) -> list:
         for M in (1, 8, 32, 128):
             a = torch.randn(M, K, generator=_gen(7)).half().to(dev)
             out = torch.empty((M, N), dtype=torch.float16, device=dev)
-            strips = M <= quant_linear.decode_rows(K, N)
+            first, last = quant_linear.strip_rows(K, N, True)
+            strips = M <= quant_linear.decode_rows(K, N) or first <= M <= last
+            batch = M >= _pk.strip_rows_from(N)
 
-            def step(i):  # what QuantLinear runs: the strip copy for decode rows, else blocks
+            def step(i):  # what QuantLinear runs: the strip copy up to its last row, else blocks
                 if strips:
                     _pk.w4a16_gemm_strips(a, qss[i % nrot], sss[i % nrot], 128, 1.0,
-                                          torch.float16, out=out)
+                                          torch.float16, out=out, rows=batch)
                 else:
                     _pk.w4a16_gemm(a, qts[i % nrot], scs[i % nrot], 128, 1.0, torch.float16,
                                    out=out, tiled=True)
