@@ -183,6 +183,15 @@ int v2_f8_launch(const uint8_t* a8, int64_t lda, const uint8_t* b8, int64_t ldb,
                  float out_scale, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
                  hipStream_t s);
 
+// Dense fp16 / bf16 GEMM on 128 x 256 or 64 x 256 tiles, B read by transposing LDS reads
+// (gemm_dense_tr.hip): N % 256 == 0, K % (64 * split) == 0; split > 1 writes fp32 partial planes to
+// `partials` and reduces them.
+bool dense_tr_ok(int M, int N, int K, int split, int64_t lda, const void* b, int64_t ldb,
+                 int64_t ldc, int c_dtype, const void* c);
+int dense_tr_launch(bool bf16, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
+                    int c_dtype, int64_t ldc, int M, int N, int K, int split, float* partials,
+                    hipStream_t s);
+
 // W4A16 GEMM with the int4 B tile kept packed in LDS and read with transposing 4-bit reads,
 // 128 x 256 tiles, eight waves splitting each k-tile in halves (w4a16_tr4.hip); N % 256 == 0,
 // K % (128 * split) == 0; split > 1 writes fp32 partial planes and reduces them.

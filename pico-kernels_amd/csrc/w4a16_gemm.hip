@@ -358,6 +358,9 @@ int gemm_launch(const GemmPlan& pl, int bmode, const void* a, int64_t lda, const
                 int64_t ldb, const void* scales, int group, OutEpi epi, void* c,
                 int c_dtype, int64_t ldc, int M, int N, int K, void* workspace, hipStream_t s,
                 bool partials_only) {
+  if (bmode != kBInt4 && dense_tr_ok(M, N, K, pl.split, lda, b, ldb, ldc, c_dtype, c))
+    return dense_tr_launch(bmode == kBDenseBF16, a, lda, b, ldb, c, c_dtype, ldc, M, N, K, pl.split,
+                           pl.split > 1 ? split_partials(workspace, false) : nullptr, s);
   // 128/256-row tiles: the large-tile 32x32-MFMA kernel when its constraints hold.
   if (pl.cfg.bm >= 128 &&
       v2_f16_ok(M, N, K, pl.k_slice, group, scales != nullptr, lda, ldb, bmode == kBInt4))
