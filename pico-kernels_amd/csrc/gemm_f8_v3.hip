@@ -100,7 +100,8 @@ __device__ __forceinline__ void f8_static_for(F&& f) {
   }
 }
 
-template <int BLAYOUT, int BN>
+// EDGE: fewer than 256 rows, or K not a multiple of 128 (see the DMA sources).
+template <int BLAYOUT, int BN, bool EDGE>
 __global__ __launch_bounds__(512) void gemm_f8_v3_kernel(F8Params p) {
   constexpr int BM = 256, BK = 64;
   constexpr int WAVES_N = BN / 64, WAVES_M = 8 / WAVES_N;
@@ -126,27 +127,35 @@ __global__ __launch_bounds__(512) void gemm_f8_v3_kernel(F8Params p) {
   f8_tile_of<BN == 128 ? 2 : 4>(blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn);
   // The last row of tiles ends at row M (M >= BM): where M % BM != 0 it overlaps the row of
   // tiles before it, whose rows it computes to the same bits, so no A row past M is read.
-  const int m0 = min(tm * BM, p.M - BM), n0 = tn * BN;
-  const int ktiles = p.K / BK;
+  // Fewer than BM rows (EDGE): row M - 1 stands in for the rows past it.
+  const int m0 = EDGE ? max(min(tm * BM, p.M - BM), 0) : min(tm * BM, p.M - BM), n0 = tn * BN;
+  const int ktiles = (p.K + BK - 1) / BK;
 
   // ---- DMA sources. A: NAD = 4 1 KB instructions per wave and k-tile pair, instruction i
   // rows (4 wave + i) * 8 .. +7 of 128 bytes (lane L: row + L / 8, slot L % 8 holding chunk
   // (L % 8) ^ ((row >> 1) & 7)); instructions 2 and 3 are 0 and 1 sixteen rows on (the same
   // chunk pattern), by the scalar offset. Every row read is < M (the tile row above) and
   // every k < K (K % 128 == 0: whole pairs), so no access depends on how the hardware
-  // range-checks the scalar offset. B: NBD per wave and k-tile ----
+  // range-checks the scalar offset. B: NBD per wave and k-tile.
+  // EDGE: each instruction has a lane offset of its own, its row clamped to M - 1, and what lies
+  // past K (whole 16-byte chunks of A and (N, K) B, K % 16 == 0; whole rows of (K, N) B) is asked
+  // for at a lane offset past the buffer, which reads nothing and fills LDS with zeros. These
+  // selects (and four more registers) cost the other shapes 2-3%: a variant of its own ----
   static_assert(NAD == 4, "four A instructions per wave and pair");
+  constexpr int kPast = -16;  // as an unsigned offset beyond every buffer
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda));
-  int a_off[2];
+  constexpr int NAO = EDGE ? NAD : 2;
+  int a_off[NAO], a_k[2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < NAO; ++i) {
     const int r = (wave * NAD + i) * 8 + (lane >> 3);
     const int c = (lane & 7) ^ ((r >> 1) & 7);
-    a_off[i] = (int)((int64_t)(m0 + r) * p.lda) + c * 16;
+    a_off[i] = (int)((int64_t)(EDGE ? min(m0 + r, p.M - 1) : m0 + r) * p.lda) + c * 16;
+    if (i < 2) a_k[i] = c * 16;
   }
   const int a_skip = 16 * (int)p.lda;  // bytes of 16 rows
   __amdgpu_buffer_rsrc_t rb;
-  int b_off[NBD];
+  int b_off[NBD], b_k[NBD];
   if constexpr (BLAYOUT == 1) {
     rb = make_rsrc(p.b, (uint32_t)((int64_t)p.N * p.ldb));
 #pragma unroll
@@ -154,6 +163,7 @@ __global__ __launch_bounds__(512) void gemm_f8_v3_kernel(F8Params p) {
       const int r = (wave * NBD + i) * 16 + (lane >> 2);
       const int c = (lane & 3) ^ ((r >> 2) & 3);
       b_off[i] = (int)((int64_t)min(n0 + r, p.N - 1) * p.ldb) + c * 16;
+      b_k[i] = c * 16;
     }
   } else {
     rb = make_rsrc(p.b, (uint32_t)((int64_t)p.K * p.ldb));
@@ -163,18 +173,25 @@ __global__ __launch_bounds__(512) void gemm_f8_v3_kernel(F8Params p) {
       const int k = (wave * NBD + i) * (64 / CPR) + lane / CPR;  // 1 KB of k rows per instruction
       const int c = BN == 256 ? (lane & 15) ^ (2 * (k & 7)) : (lane & 7) ^ (k & 7);
       b_off[i] = (int)((int64_t)k * p.ldb) + min(n0 + c * 16, p.N - 16);
+      b_k[i] = k;
     }
   }
   // B of k-tile kt; A of k-tile pair kp (k-tiles 2 kp, 2 kp + 1).
   auto issue_b = [&](int kt, char* sB) {
     const int bs = BLAYOUT == 1 ? kt * BK : (int)((int64_t)kt * BK * p.ldb);
 #pragma unroll
-    for (int i = 0; i < NBD; ++i) f8_dma16(rb, sB + (wave * NBD + i) * 1024, b_off[i], bs);
+    for (int i = 0; i < NBD; ++i)
+      f8_dma16(rb, sB + (wave * NBD + i) * 1024, !EDGE || b_k[i] < p.K - kt * BK ? b_off[i] : kPast, bs);
   };
   auto issue_a = [&](int kp, char* sAP) {
 #pragma unroll
-    for (int i = 0; i < NAD; ++i)
-      f8_dma16(ra, sAP + (wave * NAD + i) * 1024, a_off[i & 1], kp * 2 * BK + (i >> 1) * a_skip);
+    for (int i = 0; i < NAD; ++i) {
+      if constexpr (EDGE)
+        f8_dma16(ra, sAP + (wave * NAD + i) * 1024,
+                 a_k[i & 1] < p.K - kp * 2 * BK ? a_off[i] : kPast, kp * 2 * BK);
+      else
+        f8_dma16(ra, sAP + (wave * NAD + i) * 1024, a_off[i & 1], kp * 2 * BK + (i >> 1) * a_skip);
+    }
   };
 
   // ---- fragment offsets. A, in a pair buffer: row r, 16-byte chunk c of k-tile half hf at
@@ -419,7 +436,7 @@ __global__ __launch_bounds__(512) void gemm_f8_v3_kernel(F8Params p) {
 }
 
 bool f8_v3_ok(int M, int N, int K, int64_t lda, int64_t ldb, int b_layout, const void* b) {
-  if (M < 256 || N < 256 || K % 128 || N % 16 || lda % 16 || ldb % 16) return false;
+  if (N < 16 || K % 16 || N % 16 || lda % 16 || ldb % 16) return false;
   if ((reinterpret_cast<uintptr_t>(b) & 15) != 0) return false;
   if ((int64_t)M * lda >= (1ll << 31)) return false;
   return (b_layout == 1 ? (int64_t)N * ldb : (int64_t)K * ldb) < (1ll << 31);
@@ -451,13 +468,20 @@ int f8_v3_launch(const uint8_t* a8, int64_t lda, const uint8_t* b8, int64_t ldb,
   const bool narrow = (int64_t)p.tiles_m * cdiv(N, 256) < cus;
   p.tiles_n = (int)cdiv(N, narrow ? 128 : 256);
   const dim3 grid(p.tiles_m * p.tiles_n);
-  if (narrow) {
-    if (b_layout == 1) gemm_f8_v3_kernel<1, 128><<<grid, 512, 0, s>>>(p);
-    else gemm_f8_v3_kernel<0, 128><<<grid, 512, 0, s>>>(p);
-  } else {
-    if (b_layout == 1) gemm_f8_v3_kernel<1, 256><<<grid, 512, 0, s>>>(p);
-    else gemm_f8_v3_kernel<0, 256><<<grid, 512, 0, s>>>(p);
-  }
+  const bool edge = M < 256 || K % 128 != 0;
+  auto go = [&](auto L, auto BN, auto E) {
+    gemm_f8_v3_kernel<decltype(L)::value, decltype(BN)::value, decltype(E)::value != 0><<<grid, 512, 0, s>>>(p);
+  };
+  auto by_edge = [&](auto L, auto BN) {
+    if (edge) go(L, BN, pk_int_c<1>{});
+    else go(L, BN, pk_int_c<0>{});
+  };
+  auto by_tile = [&](auto L) {
+    if (narrow) by_edge(L, pk_int_c<128>{});
+    else by_edge(L, pk_int_c<256>{});
+  };
+  if (b_layout == 1) by_tile(pk_int_c<1>{});
+  else by_tile(pk_int_c<0>{});
   PK_LAUNCH_CHECK("fp8 gemm (v3)");
   return PK_OK;
 }

@@ -1,23 +1,23 @@
-// Large-tile MFMA GEMMs for gfx950: W4A16 / dense fp16 (v_mfma_f32_32x32x16_f16) and
-// e4m3 fp8 (v_mfma_f32_32x32x64_f8f6f4).
+// Large-tile MFMA GEMM for gfx950: W4A16 and dense 16-bit (v_mfma_f32_32x32x16_f16 / _bf16), for
+// the shapes and operands that the packed-B GEMM and the dense GEMM by transposing reads leave.
 //
-// Design (f16: 8 waves, two per SIMD: 256 x 128 tiles as 4 x 2 waves of 64 x 64, 128 x 128
-// tiles as 2 x 4 waves of 64 x 32; fp8 256 x 256: 8 waves, 2 x 4, each a 128 x 64 block):
-//  * LDS tiles are rows of 128 bytes (64 fp16 or 128 fp8 values of k) in 8 chunks of 16 B;
-//    chunk c of row r is stored in slot c ^ ((r >> 1) & 7). Sixteen lanes reading 16
-//    consecutive rows at one chunk then touch 16 distinct 16-byte bank groups.
-//  * A (and a (N, K) fp8 B) go global -> LDS by buffer DMA (buffer_load ... lds): no VGPR
-//    staging, no ds_write. Each pipeline stage is its own __shared__ array so the compiler's
-//    wait-count insertion only waits for DMA into the stage being read.
+// Design (8 waves, two per SIMD: 256 x 128 tiles as 4 x 2 waves of 64 x 64, 128 x 128 tiles as
+// 2 x 4 waves of 64 x 32):
+//  * LDS tiles are rows of 128 bytes (64 values of k) in 8 chunks of 16 B; chunk c of row r is
+//    stored in slot c ^ ((r >> 1) & 7). Sixteen lanes reading 16 consecutive rows at one chunk
+//    then touch 16 distinct 16-byte bank groups.
+//  * A goes global -> LDS by buffer DMA (buffer_load ... lds): no VGPR staging, no ds_write. Each
+//    pipeline stage is its own __shared__ array so the compiler's wait-count insertion only
+//    waits for DMA into the stage being read.
 //  * int4 B is loaded into registers, dequantised (exact codes via the 0x6400 fp16 exponent
-//    trick, times the fp16 group scale) and written k-contiguous; (K, N) fp16/fp8 B is
+//    trick, times the fp16 group scale) and written k-contiguous; (K, N) 16-bit B is
 //    transposed with byte permutes on the same path.
 //  * Pipelining: the loads of later tiles are issued before the MFMAs of tile t and
-//    consumed after them (three stages for f16, two for fp8); one barrier per tile.
+//    consumed after them (three stages); one barrier per tile.
 //  * Addresses: one buffer resource per operand, per-lane byte offsets computed once, the K
 //    advance folded into the scalar offset. Rows/columns past the matrix are clamped to the
 //    last valid one (never read out of bounds); their results are not stored.
-//  * Epilogue (f16 kernel): each wave stages its block of C (or of the split-K partials) in a
+//  * Epilogue: each wave stages its block of C (or of the split-K partials) in a
 //    free stage array and stores it back row-contiguous, whole 128-byte lines per store
 //    instruction.
 #include "pk_internal.h"
@@ -58,11 +58,11 @@ __device__ __forceinline__ void v2_tile_of(int bid, int tiles_m, int tiles_n, in
 struct V2Params {
   const void* a;
   int64_t lda;            // elements
-  const void* b;          // int4 words / fp16 / fp8
+  const void* b;          // int4 words / 16-bit elements
   int64_t ldb;            // words (int4) or elements
   const pk_half* scales;  // int4 group scales (K/G, N) or null
   int group;
-  OutEpi epi;             // epilogue: tensor scale / fp8 out_scale, optional bias
+  OutEpi epi;             // epilogue: tensor scale, optional bias
   void* c;
   int c_dtype;
   int64_t ldc;
@@ -462,209 +462,6 @@ void gemm_v3_f16_kernel(V2Params p) {
 }
 
 // ---------------------------------------------------------------------------------------
-// fp8 MFMA kernel (A e4m3 (M, K); B e4m3 (K, N) or (N, K)); BK = 128.
-// ---------------------------------------------------------------------------------------
-template <int BM, int BN, int WAVES_M, int WAVES_N, int BLAYOUT>
-__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_v2_f8_kernel(V2Params p) {
-  constexpr int NW = WAVES_M * WAVES_N, T = 64 * NW;
-  constexpr int WTM = BM / WAVES_M, WTN = BN / WAVES_N;
-  constexpr int FM = WTM / 32, FN = WTN / 32;
-  constexpr int A_DMA = BM / (8 * NW), B_DMA = BN / (8 * NW);
-  constexpr int BCG = BN / 16;           // (K,N): 16-byte column groups
-  constexpr int BROWS = T / BCG;         // row groups
-  constexpr int RPT = 128 / BROWS;       // k rows per thread
-  static_assert(RPT == 8 || RPT == 4, "(K,N) loader handles 8 or 4 rows per thread");
-
-  __shared__ __align__(16) char sA0[BM * 128];
-  __shared__ __align__(16) char sA1[BM * 128];
-  __shared__ __align__(16) char sB0[BN * 128];
-  __shared__ __align__(16) char sB1[BN * 128];
-
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm0 = (wave / WAVES_N) * WTM, wn0 = (wave % WAVES_N) * WTN;
-  int tm, tn;
-  v2_tile_of(blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int ktiles = p.K / 128;
-
-  const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda));
-  int a_off[A_DMA];
-#pragma unroll
-  for (int i = 0; i < A_DMA; ++i) {
-    const int r = (wave * A_DMA + i) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
-    a_off[i] = (int)((int64_t)min(m0 + r, p.M - 1) * p.lda) + c * 16;
-  }
-  auto issue_a = [&](int kt, char* sA) {
-#pragma unroll
-    for (int i = 0; i < A_DMA; ++i)
-      dma16(ra, sA + (wave * A_DMA + i) * 1024, a_off[i], kt * 128);
-  };
-
-  // B (N, K): DMA like A. B (K, N): RPT rows x 16 bytes per thread through registers.
-  __amdgpu_buffer_rsrc_t rb;
-  int b_off[BLAYOUT == 1 ? B_DMA : 1];
-  const int brg = t % BROWS, bcg = t / BROWS;
-  const int bn = min(n0 + bcg * 16, p.N - 16);
-  if (BLAYOUT == 1) {
-    rb = make_rsrc(p.b, (uint32_t)((int64_t)p.N * p.ldb));
-#pragma unroll
-    for (int i = 0; i < B_DMA; ++i) {
-      const int r = (wave * B_DMA + i) * 8 + (lane >> 3);
-      const int c = (lane & 7) ^ ((r >> 1) & 7);
-      b_off[i] = (int)((int64_t)min(n0 + r, p.N - 1) * p.ldb) + c * 16;
-    }
-  } else {
-    rb = make_rsrc(p.b, (uint32_t)((int64_t)p.K * p.ldb));
-    b_off[0] = (int)((int64_t)brg * RPT * p.ldb + bn);
-  }
-  pk_u4v breg[BLAYOUT == 0 ? RPT : 1];
-  auto issue_b = [&](int kt, char* sB) {
-    if (BLAYOUT == 1) {
-#pragma unroll
-      for (int i = 0; i < B_DMA; ++i)
-        dma16(rb, sB + (wave * B_DMA + i) * 1024, b_off[i], kt * 128);
-    } else {
-      const int soff = (int)((int64_t)kt * 128 * p.ldb);
-#pragma unroll
-      for (int r = 0; r < RPT; ++r)
-        breg[r] = __builtin_amdgcn_raw_buffer_load_b128(rb, b_off[0] + (int)(r * p.ldb), soff, 0);
-    }
-  };
-  // (K, N) B: RPT (8 or 4) rows x 16 bytes -> 16 columns x RPT k bytes, swizzled [n][k] LDS.
-  auto tr4 = [](const uint32_t in[4], uint32_t out[4]) {  // 4x4 byte transpose
-    const uint32_t t01a = __builtin_amdgcn_perm(in[1], in[0], 0x05010400u);
-    const uint32_t t01b = __builtin_amdgcn_perm(in[1], in[0], 0x07030602u);
-    const uint32_t t23a = __builtin_amdgcn_perm(in[3], in[2], 0x05010400u);
-    const uint32_t t23b = __builtin_amdgcn_perm(in[3], in[2], 0x07030602u);
-    out[0] = __builtin_amdgcn_perm(t23a, t01a, 0x05040100u);
-    out[1] = __builtin_amdgcn_perm(t23a, t01a, 0x07060302u);
-    out[2] = __builtin_amdgcn_perm(t23b, t01b, 0x05040100u);
-    out[3] = __builtin_amdgcn_perm(t23b, t01b, 0x07060302u);
-  };
-  auto store_b = [&](char* sB) {
-    if constexpr (BLAYOUT == 0) {
-      const int kb = RPT * brg;  // byte offset of the thread's k rows within the 128-byte row
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {  // dword d = columns 4d..4d+3
-        uint32_t lo[4], tl[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) lo[r] = breg[r][d];
-        tr4(lo, tl);
-        if constexpr (RPT == 8) {
-          uint32_t hi[4], th[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) hi[r] = breg[4 + r][d];
-          tr4(hi, th);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = bcg * 16 + 4 * d + q;
-            pk_u2v v = {tl[q], th[q]};
-            *reinterpret_cast<pk_u2v*>(sB + swz(n, kb >> 4) + (kb & 15)) = v;
-          }
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int n = bcg * 16 + 4 * d + q;
-            *reinterpret_cast<uint32_t*>(sB + swz(n, kb >> 4) + (kb & 15)) = tl[q];
-          }
-        }
-      }
-    }
-  };
-
-  // operand offsets: per fragment, per k64 step, two 16-byte chunks (the lane's 32 bytes)
-  int aoff[FM][2], boff[FN][2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-#pragma unroll
-    for (int i = 0; i < FM; ++i) aoff[i][ks] = swz(wm0 + 32 * i + (lane & 31), 4 * ks + 2 * (lane >> 5));
-#pragma unroll
-    for (int j = 0; j < FN; ++j) boff[j][ks] = swz(wn0 + 32 * j + (lane & 31), 4 * ks + 2 * (lane >> 5));
-  }
-  // the second chunk (c + 1) of a row r sits at slot (c + 1) ^ s = (c ^ s) ^ 1 for even c
-  auto chunk2 = [](int off) { return off ^ 16; };
-
-  pk_f16v acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = (pk_f16v){};
-
-  auto compute = [&](const char* sA, const char* sB) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      pk_i8v bf[FN];
-#pragma unroll
-      for (int j = 0; j < FN; ++j) {
-        const pk_u4v x0 = *reinterpret_cast<const pk_u4v*>(sB + boff[j][ks]);
-        const pk_u4v x1 = *reinterpret_cast<const pk_u4v*>(sB + chunk2(boff[j][ks]));
-        bf[j] = (pk_i8v){(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
-      }
-#pragma unroll
-      for (int i = 0; i < FM; ++i) {
-        const pk_u4v x0 = *reinterpret_cast<const pk_u4v*>(sA + aoff[i][ks]);
-        const pk_u4v x1 = *reinterpret_cast<const pk_u4v*>(sA + chunk2(aoff[i][ks]));
-        const pk_i8v af = {(int)x0[0], (int)x0[1], (int)x0[2], (int)x0[3], (int)x1[0], (int)x1[1], (int)x1[2], (int)x1[3]};
-#pragma unroll
-        for (int j = 0; j < FN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af, acc[i][j], 0, 0, 0, 0, 0, 0);
-      }
-    }
-  };
-
-  issue_a(0, sA0);
-  issue_b(0, sB0);
-  store_b(sB0);
-  __syncthreads();
-  int kt = 0;
-  // Scheduling barriers pin the next tile's loads at the top of each step (the compiler
-  // otherwise issues them after the MFMAs, just before the barrier that waits for them).
-  for (; kt + 1 < ktiles; kt += 2) {
-    issue_b(kt + 1, sB1);
-    issue_a(kt + 1, sA1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(sA0, sB0);
-    __builtin_amdgcn_sched_barrier(0);
-    store_b(sB1);
-    __syncthreads();
-    const int n2 = min(kt + 2, ktiles - 1);
-    issue_b(n2, sB0);
-    issue_a(n2, sA0);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(sA1, sB1);
-    __builtin_amdgcn_sched_barrier(0);
-    store_b(sB0);
-    __syncthreads();
-  }
-  if (kt < ktiles) compute(sA0, sB0);
-  mfma_drain();
-
-  // epilogue: fragments hold C^T (B is the first MFMA operand), so each register quad is
-  // four consecutive columns of one row -> one 8- or 16-byte store
-  const int esz = p.c_dtype == PK_F32 ? 4 : 2;
-  const bool vec = p.ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(p.c) & (4 * esz - 1)) == 0;
-  const int em = lane & 31, en = 4 * (lane >> 5);
-  with_dtype(p.c_dtype, [&](auto DT) {
-    constexpr int dt = decltype(DT)::value;
-#pragma unroll
-    for (int i = 0; i < FM; ++i)
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int gm = m0 + wm0 + 32 * i + em;
-          const int gn = n0 + wn0 + 32 * j + 8 * q + en;  // N % 16 == 0: all four in or out
-          if (gm < p.M && gn < p.N) {
-            pk_f4 v = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-            v = p.epi(v, gn);
-            store4_as<dt>(p.c, (int64_t)gm * p.ldc + gn, v, vec);
-          }
-        }
-  });
-}
-
-// ---------------------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------------------
 bool v2_f16_ok(int M, int N, int K, int k_slice, int group, bool has_gs, int64_t lda, int64_t ldb,
@@ -714,29 +511,6 @@ int v2_f16_launch(int bm, int bmode, const void* a, int64_t lda, const void* b, 
   }
   PK_LAUNCH_CHECK("gemm v2 f16");
   if (split > 1 && !partials_only) return splitk_reduce(p.partials, split, M, N, epi, c, c_dtype, ldc, s);
-  return PK_OK;
-}
-
-int v2_f8_launch(const uint8_t* a8, int64_t lda, const uint8_t* b8, int64_t ldb, int b_layout,
-                 float out_scale, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
-                 hipStream_t s) {
-  V2Params p;
-  p.a = a8; p.lda = lda; p.b = b8; p.ldb = ldb; p.scales = nullptr; p.group = K;
-  p.epi = OutEpi(out_scale); p.c = c; p.c_dtype = c_dtype; p.ldc = ldc;
-  p.M = M; p.N = N; p.K = K; p.split = 1; p.k_slice = K; p.partials = nullptr;
-  const bool big = (int64_t)M * N >= (int64_t)2048 * 2048;
-  const int bm = big ? 256 : 128, bn = big ? 256 : 128;
-  p.tiles_m = (int)cdiv(M, bm);
-  p.tiles_n = (int)cdiv(N, bn);
-  const int grid = p.tiles_m * p.tiles_n;
-  if (big) {
-    if (b_layout == 1) gemm_v2_f8_kernel<256, 256, 2, 4, 1><<<grid, 512, 0, s>>>(p);
-    else gemm_v2_f8_kernel<256, 256, 2, 4, 0><<<grid, 512, 0, s>>>(p);
-  } else {
-    if (b_layout == 1) gemm_v2_f8_kernel<128, 128, 2, 2, 1><<<grid, 256, 0, s>>>(p);
-    else gemm_v2_f8_kernel<128, 128, 2, 2, 0><<<grid, 256, 0, s>>>(p);
-  }
-  PK_LAUNCH_CHECK("gemm v2 fp8");
   return PK_OK;
 }
 

@@ -179,10 +179,6 @@ int v2_f16_launch(int bm, int bmode, const void* a, int64_t lda, const void* b, 
                   const void* scales, int group, OutEpi epi, void* c, int c_dtype, int64_t ldc,
                   int M, int N, int K, int split, void* workspace, hipStream_t s,
                   bool partials_only);
-int v2_f8_launch(const uint8_t* a8, int64_t lda, const uint8_t* b8, int64_t ldb, int b_layout,
-                 float out_scale, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
-                 hipStream_t s);
-
 // Dense fp16 / bf16 GEMM on 128 x 256 or 64 x 256 tiles, B read by transposing LDS reads
 // (gemm_dense_tr.hip): N % 256 == 0, K % (64 * split) == 0; split > 1 writes fp32 partial planes to
 // `partials` and reduces them.
@@ -204,8 +200,8 @@ int tr4_launch(const void* a, int64_t lda, const void* b, int64_t ldb, const voi
                int group, OutEpi epi, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
                int split, void* workspace, hipStream_t s, bool partials_only, bool tiled = false);
 
-// 256 x 256 fp8 GEMM with a 4-stage DMA pipeline and transposing LDS reads for (K, N) B
-// (gemm_f8_v3.hip).
+// fp8 GEMM of 256 x 256 or 256 x 128 tiles with a 4-stage DMA pipeline and transposing LDS reads for
+// (K, N) B (gemm_f8_v3.hip): any M, K % 16 == 0, N % 16 == 0, 16-byte aligned rows of A and B.
 bool f8_v3_ok(int M, int N, int K, int64_t lda, int64_t ldb, int b_layout, const void* b);
 int f8_v3_launch(const uint8_t* a8, int64_t lda, const uint8_t* b8, int64_t ldb, int b_layout,
                  float out_scale, void* c, int c_dtype, int64_t ldc, int M, int N, int K,
