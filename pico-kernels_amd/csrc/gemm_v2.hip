@@ -90,7 +90,9 @@ enum V2B { kV2Int4 = 0, kV2F16KN = 1, kV2BF16KN = 2 };  // B (K, N): int4 words,
 // NWM x NWN waves, two per SIMD (measured on MI355X: one wave per SIMD reads LDS at ~96 B/clk
 // per CU, two at ~170): BM = 256 as 4 x 2 waves of 64 x 64; BM = 128 as 2 x 4 waves of 64 x 32
 // for M <= 128, where 256-row tiles would leave half the MFMA work on padding rows.
-template <int BMODE, bool GS, int BM, int NWM, int NWN>
+// KTAIL (int4 without group scales, unsplit): K is not a multiple of 64. What the last k-tile holds
+// past K is asked for at lane offsets past the buffers, which reads nothing and gives zeros.
+template <int BMODE, bool GS, int BM, int NWM, int NWN, bool KTAIL = false>
 __global__ __launch_bounds__(64 * NWM * NWN)
 __attribute__((amdgpu_waves_per_eu(NWM * NWN / 4, NWM * NWN / 4)))
 void gemm_v3_f16_kernel(V2Params p) {
@@ -114,21 +116,25 @@ void gemm_v3_f16_kernel(V2Params p) {
   v2_tile_of(blockIdx.x, p.tiles_m, p.tiles_n, &tm, &tn);
   const int m0 = tm * BM, n0 = tn * BN;
   const int k_begin = blockIdx.y * p.k_slice;
-  const int ktiles = p.k_slice / 64;
+  static_assert(!KTAIL || (BMODE == kV2Int4 && !GS), "K tails: per-tensor int4");
+  const int ktiles = KTAIL ? (p.K + 63) / 64 : p.k_slice / 64;
   const int last = ktiles - 1;
+  constexpr int kPast = -16;  // as an unsigned offset beyond every buffer
 
   const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.a, (uint32_t)((int64_t)p.M * p.lda * 2));
-  int a_off[A_DMA];
+  int a_off[A_DMA], a_k[2];
 #pragma unroll
   for (int i = 0; i < A_DMA; ++i) {
     const int r = (wave * A_DMA + i) * 8 + (lane >> 3);
-    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);  // of instruction i + 2 as of i
     a_off[i] = (int)((int64_t)min(m0 + r, p.M - 1) * p.lda * 2) + c * 16;
+    if (i < 2) a_k[i] = c * 8;
   }
+  auto a_voff = [&](int kt, int i) { return !KTAIL || a_k[i & 1] < p.K - kt * 64 ? a_off[i] : kPast; };
   auto issue_a = [&](int kt, char* sA) {
     const int soff = (k_begin + kt * 64) * 2;
 #pragma unroll
-    for (int i = 0; i < A_DMA; ++i) dma16(ra, sA + (wave * A_DMA + i) * 1024, a_off[i], soff);
+    for (int i = 0; i < A_DMA; ++i) dma16(ra, sA + (wave * A_DMA + i) * 1024, a_voff(kt, i), soff);
   };
 
   const int brg = t % BROWS, bcg = t / BROWS;
@@ -146,6 +152,9 @@ void gemm_v3_f16_kernel(V2Params p) {
       make_rsrc(p.scales, has_gs ? (uint32_t)((int64_t)(p.K / p.group) * p.N * 2) : 16u);
   uint32_t breg[3][RPT][4];
   pk_u4v sreg[3] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+  auto b_voff = [&](int kt, int r) {  // int4 row r of the lane's
+    return !KTAIL || brg * RPT + r < p.K - kt * 64 ? b_off + (int)(r * p.ldb * 4) : kPast;
+  };
   auto load_b = [&](int kt, auto SLOT) {
     constexpr int sl = decltype(SLOT)::value;
     const int k0 = k_begin + kt * 64;
@@ -153,7 +162,7 @@ void gemm_v3_f16_kernel(V2Params p) {
       const int soff = (int)((int64_t)k0 * p.ldb * 4);
 #pragma unroll
       for (int r = 0; r < RPT; ++r)
-        breg[sl][r][0] = __builtin_amdgcn_raw_buffer_load_b32(rb, b_off + (int)(r * p.ldb * 4), soff, 0);
+        breg[sl][r][0] = __builtin_amdgcn_raw_buffer_load_b32(rb, b_voff(kt, r), soff, 0);
       if constexpr (has_gs) sreg[sl] = __builtin_amdgcn_raw_buffer_load_b128(rs, bn * 2, (k0 / p.group) * p.N * 2, 0);
     } else {
       const int soff = (int)((int64_t)k0 * p.ldb * 2);
@@ -168,7 +177,7 @@ void gemm_v3_f16_kernel(V2Params p) {
   auto load_b_row = [&](int kt, auto SLOT, int r) {
     constexpr int sl = decltype(SLOT)::value;
     const int k0 = k_begin + kt * 64;
-    breg[sl][r][0] = __builtin_amdgcn_raw_buffer_load_b32(rb, b_off + (int)(r * p.ldb * 4), (int)((int64_t)k0 * p.ldb * 4), 0);
+    breg[sl][r][0] = __builtin_amdgcn_raw_buffer_load_b32(rb, b_voff(kt, r), (int)((int64_t)k0 * p.ldb * 4), 0);
     if constexpr (has_gs) {
       if (r == 0) sreg[sl] = __builtin_amdgcn_raw_buffer_load_b128(rs, bn * 2, (k0 / p.group) * p.N * 2, 0);
     }
@@ -245,7 +254,7 @@ void gemm_v3_f16_kernel(V2Params p) {
     const int soff = (k_begin + kt * 64) * 2;
 #pragma unroll
     for (int i = 0; i < A_DMA; ++i)
-      if (i * 4 / A_DMA == part) dma16(ra, sA + (wave * A_DMA + i) * 1024, a_off[i], soff);
+      if (i * 4 / A_DMA == part) dma16(ra, sA + (wave * A_DMA + i) * 1024, a_voff(kt, i), soff);
   };
   auto compute_store = [&](const char* sA, const char* sB, auto SLOT, char* sBn, int kta, char* sAn,
                            auto LSLOT) {
@@ -466,7 +475,9 @@ void gemm_v3_f16_kernel(V2Params p) {
 // ---------------------------------------------------------------------------------------
 bool v2_f16_ok(int M, int N, int K, int k_slice, int group, bool has_gs, int64_t lda, int64_t ldb,
                bool int4) {
-  if (M < 64 || N < 64 || N % 8 || k_slice % 64) return false;
+  if (N < 64 || N % 8) return false;
+  // int4: any M and a K of 32-row steps (an unsplit, per-tensor K may end within a k-tile)
+  if (int4 ? k_slice % 64 && (has_gs || k_slice != K) : M < 64 || k_slice % 64) return false;
   if (has_gs && group % 64) return false;
   // 32-bit buffer offsets
   if ((int64_t)M * lda * 2 >= (1ll << 31)) return false;
@@ -495,7 +506,10 @@ int v2_f16_launch(int bm, int bmode, const void* a, int64_t lda, const void* b, 
   // 64 x 32 (measured 7-14% faster on the Llama-3-8B layers at M = 64 and 128 than 2 x 2
   // waves of 64 x 64).
   if (bmode == kV2Int4) {
-    if (bm == 256) {
+    if (p.k_slice % 64) {
+      if (bm == 256) gemm_v3_f16_kernel<kV2Int4, false, 256, 4, 2, true><<<grid, 512, 0, s>>>(p);
+      else gemm_v3_f16_kernel<kV2Int4, false, 128, 2, 4, true><<<grid, 512, 0, s>>>(p);
+    } else if (bm == 256) {
       if (gs) gemm_v3_f16_kernel<kV2Int4, true, 256, 4, 2><<<grid, 512, 0, s>>>(p);
       else gemm_v3_f16_kernel<kV2Int4, false, 256, 4, 2><<<grid, 512, 0, s>>>(p);
     } else {

@@ -362,9 +362,14 @@ int gemm_launch(const GemmPlan& pl, int bmode, const void* a, int64_t lda, const
     return dense_tr_launch(bmode == kBDenseBF16, a, lda, b, ldb, c, c_dtype, ldc, M, N, K, pl.split,
                            pl.split > 1 ? split_partials(workspace, false) : nullptr, s);
   // 128/256-row tiles: the large-tile 32x32-MFMA kernel when its constraints hold.
-  if (pl.cfg.bm >= 128 &&
+  // int4 of fewer than 64 rows with K % 128 != 0 (no register-dequant kernel, no even split): 128-row
+  // tiles of it as well. Measured on MI355X against this file's kernel: per-tensor 16 x 4128 x 4104
+  // 109 -> 36 us, 63 x 4128 x 4096 140 -> 39.5, 16 x 1056 x 1032 30 -> 12; with a K tail (K % 64 != 0)
+  // above 64 rows 200 x 4128 x 4096 279 -> 54, 2048 x 8160 x 8184 1075 -> 266.
+  const bool few = bmode == kBInt4 && pl.cfg.bm < 128 && K % 128 != 0 && pl.split == 1;
+  if ((pl.cfg.bm >= 128 || few) &&
       v2_f16_ok(M, N, K, pl.k_slice, group, scales != nullptr, lda, ldb, bmode == kBInt4))
-    return v2_f16_launch(pl.cfg.bm, bmode == kBInt4 ? 0 : (bmode == kBDenseBF16 ? 2 : 1), a, lda, b, ldb, scales, group,
+    return v2_f16_launch(few ? 128 : pl.cfg.bm, bmode == kBInt4 ? 0 : (bmode == kBDenseBF16 ? 2 : 1), a, lda, b, ldb, scales, group,
                          epi, c, c_dtype, ldc, M, N, K, pl.split, workspace, s,
                          partials_only);
   GemmParams p;
