@@ -185,7 +185,7 @@ def _gpu_args(what: str, first: torch.Tensor, *others: torch.Tensor | None) -> N
     dev = first.get_device() if first.is_cuda else -1
     ok = dev >= 0
     for t in others:
-        if t is not None and t.get_device() != dev:  # -1 on the host
+        if t is not None and (not t.is_cuda or t.get_device() != dev):
             ok = False
     if not ok:
         raise ValueError(f"{what}: every tensor must be on one GPU (got "
@@ -288,7 +288,9 @@ def _post_counter(device: torch.device, stream: int) -> int:
     key = (device.index, stream)
     t = _post_counters.get(key)
     if t is None:
-        t = _post_counters[key] = torch.zeros(POST_COUNTER_BYTES, dtype=torch.uint8, device=device)
+        # one tensor per key, whichever thread comes first
+        t = _post_counters.setdefault(
+            key, torch.zeros(POST_COUNTER_BYTES, dtype=torch.uint8, device=device))
     return t.data_ptr()
 
 
