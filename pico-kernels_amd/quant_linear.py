@@ -254,6 +254,16 @@ class QuantLinear(nn.Module):
                 self._fast = call
         return call
 
+    def _strip_matmul(self, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
+        """fp16 rows on the strip copy. The prepared call wants contiguous, 16-byte aligned rows;
+        a batch beyond ``decode_rows`` may have any, as the kernels on ``qweight`` take it: row
+        strides go to the kernel, other forms are copied."""
+        if x.shape[0] <= self.decode_rows or (x.is_contiguous() and x.data_ptr() % 16 == 0):
+            return self._strips_call(out_dtype)(x)
+        return _pk.w4a16_gemm_strips(x, self.qstrips, self.sstrips, self.group_size,
+                                     self._smax if self.scheme == "per_input" else 1.0, out_dtype,
+                                     bias=self.bias, rows=True)
+
     def _drop_calls(self) -> None:
         self._calls = {}
         self._fast = None
@@ -288,14 +298,18 @@ class QuantLinear(nn.Module):
         # decode fast path: fp16 rows of a group layer with a strip copy, one prepared call
         fast = self._fast
         if (fast is not None and x.dim() == 2 and x.dtype == torch.float16
-                and x.shape[1] == self.in_features and self._on_strips(x.shape[0])):
-            return fast(x)
+                and x.shape[1] == self.in_features):
+            rows = x.shape[0]
+            if rows <= self.decode_rows:
+                return fast(x)
+            if self._on_strips(rows):
+                return self._strip_matmul(x, torch.float16)
         assert x.shape[-1] == self.in_features
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
         strips = self.decode and self._on_strips(x2.shape[0])
         if x2.dtype == torch.float16 and self.scheme == "group" and strips:
-            return self._strips_call(torch.float16)(x2).view(*lead, self.out_features)
+            return self._strip_matmul(x2, torch.float16).view(*lead, self.out_features)
         out_dtype = x.dtype if x.dtype in _OUT_DTYPES else torch.float16
         # the bias is added in the matmul's epilogue (before the one rounding to out_dtype)
         if self.scheme == "per_input":
@@ -316,7 +330,7 @@ class QuantLinear(nn.Module):
     def _matmul(self, xp: torch.Tensor, strips: bool, out_dtype: torch.dtype) -> torch.Tensor:
         """fp16 rows (prepared for the scheme) times the weight, plus the bias."""
         if strips:
-            return self._strips_call(out_dtype)(xp)
+            return self._strip_matmul(xp, out_dtype)
         if self.scheme == "per_input":
             return _pk.w4a16_gemm(xp, self.qweight, None, 0, self._smax, out_dtype, bias=self.bias,
                                   tiled=self.tiled)

@@ -95,6 +95,25 @@ def test_quant_linear_batches(cuda, scheme, out_f):
                 assert torch.equal(q(x.view(2, 8, -1)).view(M, -1), y)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("out_f", [1024, 17424])
+def test_quant_linear_batch_forms(cuda, out_f):
+    """Batches in forms other than contiguous, aligned rows: a misaligned base, a row pitch that
+    is a multiple of 16 bytes or not, transposed rows; each gives the contiguous copy's bits."""
+    lin = torch.nn.Linear(256, out_f, device=cuda, dtype=torch.float16)
+    q = quant_linear.QuantLinear.from_linear(lin, 128)
+    first, _ = quant_linear.strip_rows(256, out_f, q.tiled)
+    for M in (first, 16, 32):
+        flat = torch.randn(M * 272 + 1, device=cuda).half()
+        forms = (flat[1:M * 256 + 1].view(M, 256), flat[:M * 264].view(M, 264)[:, :256],
+                 flat[:M * 264].view(M, 264)[:, 1:257], flat[:M * 257].view(M, 257)[:, :256],
+                 flat[:M * 256].view(256, M).t())
+        for x in forms:
+            assert torch.equal(q(x), q(x.clone(memory_format=torch.contiguous_format)))
+        x = forms[0].view(1, M, 256)
+        assert torch.equal(q(x)[0], q(forms[0].clone()))
+
+
 def test_rule():
     r = quant_linear.strip_rows
     assert r(4096, 8192, True) == (9, 64) and r(4096, 8208, True) == (9, 32)
