@@ -662,11 +662,12 @@ class PreparedStrips:
             self.h = None
 
     def __call__(self, a: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-        if (a.dtype != torch.float16 or a.dim() != 2 or a.shape[1] != self.K or not a.is_cuda
+        shape = a.shape
+        if (a.dtype != torch.float16 or len(shape) != 2 or shape[1] != self.K or not a.is_cuda
                 or a.get_device() != self.dev):
             raise ValueError(f"PreparedStrips: activations must be (M, {self.K}) fp16 on "
-                             f"cuda:{self.dev} (got {tuple(a.shape)} {a.dtype} on {a.device})")
-        M = a.shape[0]
+                             f"cuda:{self.dev} (got {tuple(shape)} {a.dtype} on {a.device})")
+        M = shape[0]
         if a.stride(0) != self.lda or a.stride(1) != 1 or a.data_ptr() % 16:
             a = a.contiguous() if self.lda == self.K else _rows_ok(a)
             if a.stride(0) != self.lda or a.data_ptr() % 16:

@@ -297,15 +297,16 @@ class QuantLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # decode fast path: fp16 rows of a group layer with a strip copy, one prepared call
         fast = self._fast
-        if (fast is not None and x.dim() == 2 and x.dtype == torch.float16
-                and x.shape[1] == self.in_features):
-            rows = x.shape[0]
+        shape = x.shape
+        if (fast is not None and len(shape) == 2 and x.dtype == torch.float16
+                and shape[1] == self.in_features):
+            rows = shape[0]
             if rows <= self.decode_rows:
                 return fast(x)
             if self._on_strips(rows):
                 return self._strip_matmul(x, torch.float16)
-        assert x.shape[-1] == self.in_features
-        lead = x.shape[:-1]
+        assert shape[-1] == self.in_features
+        lead = shape[:-1]
         x2 = x.reshape(-1, self.in_features)
         strips = self.decode and self._on_strips(x2.shape[0])
         if x2.dtype == torch.float16 and self.scheme == "group" and strips:
