@@ -629,7 +629,7 @@ class PreparedStrips:
     row stride ``lda`` (elements; default K). The tensors stay referenced here, and must stay
     in place, while the object lives (QuantLinear drops it when its buffers move or change)."""
 
-    __slots__ = ("h", "N", "K", "lda", "out_dtype", "dev", "run", "run_rows", "rows_from",
+    __slots__ = ("h", "N", "K", "lda", "strides", "out_dtype", "dev", "run", "run_rows", "rows_from",
                  "run_events", "release", "_keep")
 
     def __init__(self, qstrips: torch.Tensor, sstrips: torch.Tensor | None, group_size: int,
@@ -639,6 +639,7 @@ class PreparedStrips:
         self.K, W = qstrips.shape
         self.N = 8 * W
         self.lda = self.K if lda is None else int(lda)
+        self.strides = (self.lda, 1)
         self.out_dtype = out_dtype
         self.dev = qstrips.device.index
         self._keep = (qstrips, sstrips, bias)
@@ -668,20 +669,25 @@ class PreparedStrips:
             raise ValueError(f"PreparedStrips: activations must be (M, {self.K}) fp16 on "
                              f"cuda:{self.dev} (got {tuple(shape)} {a.dtype} on {a.device})")
         M = shape[0]
-        if a.stride(0) != self.lda or a.stride(1) != 1 or a.data_ptr() % 16:
+        ptr = a.data_ptr()
+        if a.stride() != self.strides or ptr & 15:
             a = a.contiguous() if self.lda == self.K else _rows_ok(a)
             if a.stride(0) != self.lda or a.data_ptr() % 16:
                 raise ValueError(f"PreparedStrips: activations need row stride {self.lda}, "
                                  "16-byte aligned")
+            ptr = a.data_ptr()
         if out is None:
-            out = a.new_empty((M, self.N), dtype=self.out_dtype)
+            ldc = self.N
+            out = a.new_empty((M, ldc), dtype=self.out_dtype)
         elif (out.dtype != self.out_dtype or out.dim() != 2 or out.shape[0] != M
               or out.shape[1] != self.N or out.stride(1) != 1 or not out.is_cuda
               or out.get_device() != self.dev):
             raise ValueError(f"PreparedStrips: out must be ({M}, {self.N}) {self.out_dtype} with "
                              f"unit column stride on cuda:{self.dev}")
+        else:
+            ldc = out.stride(0)
         run = self.run if M < self.rows_from else self.run_rows
-        rc = run(self.h, a.data_ptr(), out.data_ptr(), out.stride(0), M,
+        rc = run(self.h, ptr, out.data_ptr(), ldc, M,
                  torch._C._cuda_getCurrentRawStream(self.dev))
         if rc != PK_OK:
             _check(rc, "pk_w4a16_strips_run")
