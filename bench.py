@@ -571,11 +571,10 @@ def bench_llama_sweep(dev, iters: int = 50) -> list:
         for M in (1, 8, 32, 128):
             a = torch.randn(M, K, generator=_gen(7)).half().to(dev)
             out = torch.empty((M, N), dtype=torch.float16, device=dev)
-            first, last = quant_linear.strip_rows(K, N, True)
-            strips = M <= quant_linear.decode_rows(K, N) or first <= M <= last
-            batch = M >= _pk.strip_rows_from(N)
+            strips = M <= quant_linear.decode_rows(K, N) or _pk.strip_batch(M, K, N, 128, True)
+            batch = M >= _pk.strip_rows_from(K, N, 128)
 
-            def step(i):  # what QuantLinear runs: the strip copy up to its last row, else blocks
+            def step(i):  # what QuantLinear runs: the strip copy where it serves, else blocks
                 if strips:
                     _pk.w4a16_gemm_strips(a, qss[i % nrot], sss[i % nrot], 128, 1.0,
                                           torch.float16, out=out, rows=batch)

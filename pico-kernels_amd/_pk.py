@@ -9,6 +9,7 @@ raises instead of falling back to another implementation.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import struct
 import threading
@@ -26,6 +27,7 @@ PK_F32, PK_F16, PK_BF16, PK_E4M3, PK_I8, PK_U8, PK_I32 = range(7)
 _TORCH_TO_PK = {torch.float32: PK_F32, torch.float16: PK_F16, torch.bfloat16: PK_BF16}
 
 PK_OK, PK_EINVAL, PK_EUNSUPPORTED, PK_EWORKSPACE, PK_EHIP = 0, -1, -2, -3, -4
+PLAN_PACKED_B = 4  # pk_w4a16_plan's id of the packed-B GEMM
 
 KERNEL_GEMV, KERNEL_GEMM, KERNEL_SKINNY, KERNEL_GEMM_TR4 = 1, 2, 3, 4  # pk_w4a16_plan kernel ids
 
@@ -428,6 +430,7 @@ def w4a16_skinny_layout(cols_per_lane: int, waves: int) -> None:
     """Fix the register-dequant kernel's layout for later plans ((0, 0): automatic)."""
     _check(lib().pk_w4a16_skinny_layout(int(cols_per_lane), int(waves)), "pk_w4a16_skinny_layout")
     _ws_bytes.clear()
+    strip_batch.cache_clear()
 
 
 def w4a16_launches(M: int, N: int, K: int, group_size: int, split_k: int) -> int:
@@ -612,17 +615,80 @@ def w4a16_gemm_strips(a: torch.Tensor, qstrips: torch.Tensor, sstrips: torch.Ten
     return out
 
 
-def strip_rows_from(N: int) -> int:
-    """Rows from which a strip-layout call of N columns runs the batch kernel
-    (pk_w4a16_strips_run_rows) instead of the decode kernel: 9, or 5 where two or four strips
-    share a workgroup (more than 256 strips). Measured on MI355X at M = 8, decode / batch kernel:
-    4096 x 4096 5.8 / 5.7 us, 14336 x 4096 11.8 / 12.9; 4096 x 6144 7.5 / 6.5, 4096 x 14336
-    11.5 / 10.1, 8192 x 14336 20.0 / 15.4."""
-    return 5 if N > 16 * 256 else 9
+def strip_rows_from(K: int, N: int, group_size: int) -> int:
+    """Rows from which a strip-layout call that the decode kernel could serve (up to 8) runs the
+    batch kernel (pk_w4a16_strips_run_rows): 9, or 5 (6 up to 2048 inputs) where two or four strips
+    share a workgroup (more than 256 strips), they run in one round (at most 1024) and no group
+    ends inside a 128-row block. Measured on MI355X, decode / batch kernel: M = 8 4096 x 4096 5.8 /
+    5.7 us, 14336 x 4096 11.8 / 12.9, 4096 x 6144 7.5 / 6.5, 4096 x 14336 11.5 / 10.1, 8192 x 14336
+    20.0 / 15.4; M = 5 1280 x 12288 5.2 / 5.3, 7168 x 17408 23.3 / 25.7; groups of 32 10496 x 6144 M = 8
+    14.2 / 17.3, of 64 11264 x 10752 M = 5 21.0 / 23.8."""
+    if N <= 16 * 256 or N > 16 * 1024 or 0 < group_size < 128:
+        return 9
+    return 6 if K <= 2048 else 5
+
+
+@functools.lru_cache(maxsize=4096)
+def strip_batch(M: int, K: int, N: int, group_size: int, blocks: bool) -> bool:
+    """Whether M rows, beyond those of the decode kernel, of a layer that keeps a strip copy run
+    the batch kernel on it (pk_w4a16_gemm_strips_rows) rather than what is planned for them on
+    the row or block layout. The batch kernel's workgroups own 1, 2 or 4 strips (2 at most
+    above 32 rows) over all of K, one on a CU: it suffers where they just miss a round of 256, or
+    are few with a long K each. The other plans (pk_w4a16_plan) depend on the divisors of
+    K / 128: many short slices, or none where a prime is left, cost them up to four times.
+
+    Measured on MI355X (graphs over rotating weights; planned kernel / batch kernel in us), with
+    groups of 128 (g), 32 or 64, or one scale per tensor (t):
+      above 32 rows, packed-B GEMM planned: it fills the chip, unless K leaves it one slice.
+        8064 x 9216 g M = 64 24.0 / 41.3, 7040 x 5120 g M = 51 17.2 / 20.1; one slice: 13952 x 6144 g
+        M = 33 101 / 32.8, 9856 x 12032 g M = 64 70.3 / 50.1, but 3712 x 11520 t M = 54 21.7 / 25.5
+      above 32 rows, register-dequant kernel planned: 4096 x 14352 M = 48 g 30.8 / 24.8, t 24.2 / 25.8;
+        3072 x 8864 g M = 41 17.6 / 20.3 (277 workgroups); 11520 x 5872 t M = 33 25.1 / 28.4; few strips:
+        13312 x 1920 g M = 48 17.2 / 26.1, 9600 x 3280 t M = 36 18.6 / 20.2
+      up to 32 rows: 4096 x 14352 M = 32 g 20.9 / 14.2; few strips of a long K: 13312 x 1920 g M = 31
+        14.0 / 16.8, 8192 x 1536 g M = 11 7.7 / 8.4; 129 to 160 workgroups of four strips against a few
+        slices: 6144 x 8960 g M = 26 16.2 / 17.3; just beyond 1024 strips: 7168 x 17408 g M = 9 22.0 /
+        26.0, 5120 x 28672 g M = 16 / 17 29.1 / 24.0 and 26.2 / 28.5 (five slices, then one)."""
+    if M > 64 or M < (9 if blocks else 5):
+        return False
+    # with blocks: 4096 x 10240 M = 48 15.9 / 23.5, 8192 x 4096 M = 48 15.4 / 18.0, 14336 x 4096 M = 24
+    # 16.8 / 17.1 (a K without small divisors, 11008 x 4096 M = 32 36 / 15.5, is not told apart)
+    if blocks and M > (64 if K <= 4096 and N <= 512 * 16 else 32 if K <= 8192 else 16):
+        return False
+    kernel, split = w4a16_plan(M, N, K, group_size, 0)
+    strips, slice_rows = N // 16, K // split
+    whole = group_size >= 128  # groups of whole 128-row blocks
+    if M > 32:
+        if kernel == PLAN_PACKED_B:
+            if split == 1:
+                return strips <= (1024 if whole else 512)
+            return whole and split <= 3 and strips <= 512
+        if strips <= (128 if whole else 208) and K >= 4096 and split <= 16:
+            return False
+        if strips <= 128:
+            return K <= 6144 or slice_rows < (256 if 0 < group_size < 128 else 384)
+        if strips <= 512:
+            return whole or split >= 8 or K <= 4096
+        if slice_rows <= 256 and (whole or group_size == 0):
+            return True
+        if strips <= 1024:
+            return whole and (strips > 576 or K <= 2048) or K <= 512
+        return split >= (3 if whole else 9)
+    if strips <= (128 if K < 12288 else 192):
+        if slice_rows < 512 or K < (8192 if M <= 16 else 6400):
+            return True
+        return not (blocks or M <= 16 or K >= 12288 or 0 < group_size < 128)
+    if strips <= 1024:
+        return strips <= 512 or strips > 640 or K < 6144 or split > 3
+    if strips <= 1408:
+        return ((split >= 9 and slice_rows <= 512) or (split == 2 and K >= 3072)
+                or (not blocks and whole and split != 3))
+    return split >= 2 or (not blocks and K >= 2048)
 
 
 class PreparedStrips:
-    """``pk_w4a16_gemm_strips`` (1..8 rows) and ``pk_w4a16_gemm_strips_rows`` (5..64) bound to one strip-layout weight copy through
+    """``pk_w4a16_gemm_strips`` (1..8 rows) and ``pk_w4a16_gemm_strips_rows`` (from
+    ``strip_rows_from`` to 64) bound to one strip-layout weight copy through
     ``pk_w4a16_strips_prepare``: the fixed arguments are checked and the launches for 1..8 rows
     planned once, so a call passes only the activations, the output, the row count and the
     stream (what an eager decode loop pays per layer). Activations must be 16-byte aligned with
@@ -653,7 +719,8 @@ class PreparedStrips:
             raise PicoKernelsError("pk_w4a16_strips_prepare failed: "
                                    + L.pk_last_error().decode(errors="replace"))
         self.run, self.release = strips_run_entry(), L.pk_w4a16_strips_release
-        self.run_rows, self.rows_from = calls().pk_w4a16_strips_run_rows, strip_rows_from(self.N)
+        self.run_rows = calls().pk_w4a16_strips_run_rows
+        self.rows_from = strip_rows_from(self.K, self.N, int(group_size) if sstrips is not None else 0)
         self.run_events = L.pk_w4a16_strips_run_events
 
     def __del__(self):

@@ -32,8 +32,11 @@
 // the decode kernel) and the kernels it fell back to where the weights cannot be blocks: M = 8 /
 // 16 / 32 / 64 of 4096 x 6144 7.5 / 9.0 / 11.6 / 15.7 -> 6.5 / 6.8 / 9.2 / 13.8 us, 4096 x 4096
 // M = 16 / 32 7.2 / 9.7 -> 5.9 / 7.3, 4096 x 14336 M = 8 / 16 / 32 11.5 / 13.1 / 16.8 -> 10.1 / 10.7 /
-// 13.5, 8192 x 14336 M = 32 26.8 -> 21.4, 1024 x 2048 M = 32 7.5 -> 3.8; 11008 x 4096 (no blocks)
-// M = 32 36 -> 15.4, 2560 x 12304 28.4 -> 10.6.
+// 13.5, 8192 x 14336 M = 32 26.8 -> 21.4, 1024 x 2048 M = 32 7.5 -> 3.8; no blocks: 4096 x 14352
+// M = 32 20.9 -> 14.2, 6272 x 12304 (49 slices before) 63 -> 19. Not everywhere: where its workgroups
+// just miss a round of 256 (8064 x 9216 M = 64 24.0 -> 41.3) or are few (13312 x 1920 M = 31 14.0 -> 16.8)
+// the other kernels are the faster ones, and so is the decode kernel up to 8 rows with groups of 32
+// (10496 x 6144 14.2 -> 17.3): the callers' rules say which serves a call.
 #include "pk_internal.h"
 
 namespace pk {

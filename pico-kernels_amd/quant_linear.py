@@ -36,8 +36,8 @@ multiples of it, or per-input scales: ``QuantLinear.decode``) keep a second copy
 and group scales in the strip layout (``_pk.strip_weights`` / ``strip_scales``: each
 16-output strip's inputs contiguous), and calls of at most ``decode_rows`` rows run the
 one-launch strip kernels on it (``pk_w4a16_gemm_strips``; ``decode_rows``: 8 rows, or 4 on layers
-of more than 16384 outputs), as do batches of 9 to 16, 32 or 64 rows by the layer's shape
-(``pk_w4a16_gemm_strips_rows``; ``strip_rows``). The int4 codes are a quarter of the
+of more than 16384 outputs), as do batches of up to 64 rows where that is the faster way for the
+layer's shape (``pk_w4a16_gemm_strips_rows``; ``_pk.strip_batch``). The int4 codes are a quarter of the
 fp16 weights' bytes, so both copies together are half of them; ``decode_layout=False`` keeps
 one copy. The copies are derived buffers, outside the state dict. ``codes()`` /
 ``set_codes()``, the state dict and the file format use ``pack_int4_n`` order either way.
@@ -53,7 +53,6 @@ cast makes them). Weights need ``out % 8 == 0`` (whole int32 words) and ``in % 3
 
 from __future__ import annotations
 
-import functools
 import json
 
 import torch
@@ -84,24 +83,6 @@ def decode_rows(in_features: int, out_features: int) -> int:
     """Rows up to which a layer of this shape runs its strip copy."""
     wide = out_features // 16 > DECODE_WIDE_STRIPS
     return DECODE_MAX_ROWS_WIDE if wide else DECODE_MAX_ROWS
-
-
-@functools.lru_cache(maxsize=None)
-def strip_rows(in_features: int, out_features: int, blocks: bool) -> tuple[int, int]:
-    """(first, last) rows of a call, beyond ``decode_rows``, for which a layer of this shape runs
-    the strip copy's batch kernel (pk_w4a16_gemm_strips_rows) rather than the kernels on
-    ``qweight``: from 9 rows (5 where ``qweight`` is not in blocks) to 64 without blocks or on at
-    most 512 strips of at most 4096 inputs, to 32 up to 8192 inputs, else to 16. Measured on
-    MI355X, batch kernel against the kernels on blocks: 4096 x 4096 M = 32 / 64 7.3 / 11.6 against
-    9.6 / 13.0 us, 4096 x 10240 M = 32 / 48 13.2 / 23.5 against 19.5 / 15.9, 8192 x 4096 M = 32 / 48
-    11.8 / 18.0 against 12.1 / 15.4, 14336 x 4096 M = 16 / 24 13.5 / 17.1 against 14.2 / 16.8, 4096 x
-    17408 M = 8 / 32 17.0 / 24.0 against 15.4 / 28.2; without blocks 11008 x 4096 M = 32 15.4 against
-    36.3, 14336 x 8208 M = 64 63 against 74."""
-    if not blocks:
-        return 5, 64
-    if in_features <= 4096 and out_features <= 512 * 16:
-        return 9, 64
-    return 9, 32 if in_features <= 8192 else 16
 
 
 class QuantLinear(nn.Module):
@@ -249,6 +230,8 @@ class QuantLinear(nn.Module):
             scale = self._smax if self.scheme == "per_input" else 1.0
             call = _pk.PreparedStrips(self.qstrips, self.sstrips, self.group_size, scale, out_dtype,
                                       self.bias)
+            # beyond decode_rows _on_strips asks for the batch kernel
+            call.rows_from = min(call.rows_from, self.decode_rows + 1)
             self._calls[out_dtype] = call
             if out_dtype == torch.float16 and self.scheme == "group":
                 self._fast = call
@@ -291,8 +274,7 @@ class QuantLinear(nn.Module):
         """Whether a call of this many rows runs the strip copy (when the layer keeps it)."""
         if rows <= self.decode_rows:
             return True
-        first, last = strip_rows(self.in_features, self.out_features, self.tiled)
-        return first <= rows <= last
+        return _pk.strip_batch(rows, self.in_features, self.out_features, self.group_size, self.tiled)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # decode fast path: fp16 rows of a group layer with a strip copy, one prepared call

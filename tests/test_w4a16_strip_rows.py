@@ -63,8 +63,8 @@ def test_prepared_call_and_limits(cuda):
     qw = torch.from_numpy(oracle.pack_int4_n(codes)).to(cuda).view(torch.int32)
     qs, ss = _pk.strip_weights(qw), _pk.strip_scales(torch.from_numpy(s16).to(cuda))
     call = _pk.PreparedStrips(qs, ss, 128, 1.0, torch.float16)
-    assert call.rows_from == 5 and _pk.strip_rows_from(4096) == 9
-    for M in (5, 9, 64):
+    assert call.rows_from == _pk.strip_rows_from(512, 4352, 128)
+    for M in (6, 9, 64):
         a = torch.randn(M, 512, device=cuda).half()
         assert torch.equal(call(a), _pk.w4a16_gemm_strips(a, qs, ss, 128, 1.0, torch.float16, rows=True))
     for M in (0, 65):
@@ -83,9 +83,8 @@ def test_quant_linear_batches(cuda, scheme, out_f):
     ends, for fp16 and bf16 inputs and a 3-D input."""
     lin = torch.nn.Linear(1280, out_f, device=cuda, dtype=torch.float16)
     q = quant_linear.QuantLinear.from_linear(lin, 128, None if scheme == "group" else "rtn")
-    assert q.decode
-    first, last = quant_linear.strip_rows(1280, out_f, q.tiled)
-    for M in (1, 4, 5, 8, 9, 16, 33, last, last + 1):
+    assert q.decode and q._on_strips(9) and q._on_strips(33) and not q._on_strips(65)
+    for M in (1, 4, 5, 8, 9, 16, 33, 64, 65):
         for dt in (torch.float16, torch.bfloat16):
             x = torch.randn(M, 1280, device=cuda).to(dt)
             y = q(x)
@@ -102,8 +101,9 @@ def test_quant_linear_batch_forms(cuda, out_f):
     is a multiple of 16 bytes or not, transposed rows; each gives the contiguous copy's bits."""
     lin = torch.nn.Linear(256, out_f, device=cuda, dtype=torch.float16)
     q = quant_linear.QuantLinear.from_linear(lin, 128)
-    first, _ = quant_linear.strip_rows(256, out_f, q.tiled)
-    for M in (first, 16, 32):
+    rows = [M for M in (5, 9, 16, 32) if M > q.decode_rows and q._on_strips(M)]
+    assert len(rows) >= 2
+    for M in rows:
         flat = torch.randn(M * 272 + 1, device=cuda).half()
         forms = (flat[1:M * 256 + 1].view(M, 256), flat[:M * 264].view(M, 264)[:, :256],
                  flat[:M * 264].view(M, 264)[:, 1:257], flat[:M * 257].view(M, 257)[:, :256],
@@ -114,8 +114,38 @@ def test_quant_linear_batch_forms(cuda, out_f):
         assert torch.equal(q(x)[0], q(forms[0].clone()))
 
 
-def test_rule():
-    r = quant_linear.strip_rows
-    assert r(4096, 8192, True) == (9, 64) and r(4096, 8208, True) == (9, 32)
-    assert r(8192, 4096, True) == (9, 32) and r(8320, 4096, True) == (9, 16)
-    assert r(14336, 28672, False) == (5, 64)
+# (K, N, group (0: one scale per input), rows, whether the strip copy serves them), on both sides of
+# the rule's lines; the calls kept off the strip copy took up to 2.1 times as long on it.
+RULE = [
+    (8064, 9216, 128, 64, False), (8064, 9216, 128, 28, True),      # packed-B GEMM in 7 slices
+    (7040, 5120, 0, 35, False), (7040, 5120, 0, 32, True),
+    (13952, 6144, 128, 33, True), (9856, 12032, 128, 64, True),     # one slice
+    (3712, 11520, 0, 54, False), (3712, 11520, 128, 54, True),
+    (4096, 14352, 0, 48, False), (4096, 14352, 128, 48, True),      # register-dequant kernel
+    (13824, 8208, 0, 33, False), (6144, 8208, 0, 33, False),
+    (13312, 1920, 128, 31, False), (8192, 1536, 128, 11, False),    # few strips of a long K
+    (8192, 1536, 128, 24, False), (4096, 1536, 128, 24, True), (4096, 512, 0, 40, False),
+    (6144, 8960, 128, 26, False), (6144, 8960, 128, 10, True),      # 140 workgroups
+    (7168, 17408, 128, 9, False), (7168, 17408, 128, 32, False),    # 272 workgroups
+    (5120, 28672, 128, 16, True), (5120, 28672, 128, 17, False), (5120, 28672, 128, 8, False),
+    (768, 27136, 0, 9, False), (10368, 19200, 0, 6, False), (10368, 19200, 0, 32, False),
+    (4096, 14336, 128, 32, True), (4096, 14336, 128, 33, False), (4096, 4096, 128, 64, True),
+    (4096, 4096, 128, 65, False), (14336, 4096, 128, 16, True), (14336, 4096, 128, 17, False),
+]
+
+
+@pytest.mark.parametrize("K,N,group,rows,strips", RULE)
+def test_rule(K, N, group, rows, strips):
+    layer = quant_linear.QuantLinear(K, N, bias=False, group_size=group or 128, device="meta",
+                                     scheme="group" if group else "per_input")
+    assert layer.decode and layer._on_strips(rows) is strips
+
+
+@pytest.mark.parametrize("K,N,group,rows", [(4096, 4096, 128, 9), (4096, 4112, 128, 5), (2048, 4112, 128, 6),
+                                            (4096, 16384, 128, 5), (4096, 16400, 128, 9),
+                                            (10496, 6144, 32, 9), (11264, 10752, 64, 9),
+                                            (11264, 10752, 256, 5), (11264, 10752, 0, 5)])
+def test_rows_from(K, N, group, rows):
+    """Where the decode kernel hands over to the batch kernel: at 5..8 rows the latter takes up to
+    1.34 times as long with groups shorter than a block."""
+    assert _pk.strip_rows_from(K, N, group) == rows
