@@ -413,8 +413,8 @@ def w4a16_prep_activations(x: torch.Tensor, in_scale: torch.Tensor | None, mul: 
     the cast alone)."""
     _gpu_args("w4a16_prep_activations", x, in_scale, out)
     M, K = x.shape
-    if x.stride(1) != 1:
-        x = x.contiguous()
+    if x.stride(1) != 1 or x.stride(0) < K:
+        x = _packed_rows(x)
     if in_scale is not None:
         assert in_scale.dtype == torch.float32 and in_scale.is_contiguous() and in_scale.numel() == K
     if out is None:
@@ -479,8 +479,8 @@ class checked_activations:
             return
         _gpu_args("w4a16_prep_activations", x, in_scale)
         M, K = x.shape
-        if x.stride(1) != 1:
-            x = x.contiguous()
+        if x.stride(1) != 1 or x.stride(0) < K:
+            x = _packed_rows(x)
         if in_scale is not None:
             assert in_scale.dtype == torch.float32 and in_scale.is_contiguous() and in_scale.numel() == K
         self.out = out = torch.empty((M, K), dtype=torch.float16, device=x.device)
@@ -504,13 +504,21 @@ class checked_activations:
 
 
 def _rows_ok(t: torch.Tensor) -> torch.Tensor:
-    """Row-major with unit inner stride and 16-byte aligned rows, else a contiguous copy."""
-    es = t.element_size()
-    if (t.stride(-1) != 1 or (t.stride(0) * es) % 16 or t.data_ptr() % 16):
-        t = t.contiguous()
-        if t.data_ptr() % 16:
-            t = t.clone()
+    """Row-major with unit inner stride and 16-byte aligned rows that do not overlap, else a
+    contiguous copy."""
+    pitch, inner = t.stride()
+    if inner != 1 or (pitch * t.element_size()) % 16 or pitch < t.shape[1] or t.data_ptr() % 16:
+        t = _packed_rows(t)
     return t
+
+
+def _packed_rows(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous 16-byte aligned rows of pitch t.shape[1]: what ``contiguous`` gives, but for a
+    misaligned base and for one row (of any pitch), which it hands back as they are."""
+    t = t.contiguous()
+    if t.data_ptr() % 16:
+        return t.clone(memory_format=torch.contiguous_format)
+    return t[0].unsqueeze(0) if t.shape[0] == 1 else t
 
 
 # Workspace bytes per W4A16 shape (a pure function of the plan; cleared when the plan rules
@@ -691,8 +699,9 @@ class PreparedStrips:
     ``strip_rows_from`` to 64) bound to one strip-layout weight copy through
     ``pk_w4a16_strips_prepare``: the fixed arguments are checked and the launches for 1..8 rows
     planned once, so a call passes only the activations, the output, the row count and the
-    stream (what an eager decode loop pays per layer). Activations must be 16-byte aligned with
-    row stride ``lda`` (elements; default K). The tensors stay referenced here, and must stay
+    stream (what an eager decode loop pays per layer). Activations that are not 16-byte aligned
+    with row stride ``lda`` (elements; default K) are copied where ``lda`` is K, else refused; one
+    row may have any stride. The tensors stay referenced here, and must stay
     in place, while the object lives (QuantLinear drops it when its buffers move or change)."""
 
     __slots__ = ("h", "N", "K", "lda", "strides", "out_dtype", "dev", "run", "run_rows", "rows_from",
@@ -738,11 +747,11 @@ class PreparedStrips:
         M = shape[0]
         ptr = a.data_ptr()
         if a.stride() != self.strides or ptr & 15:
-            a = a.contiguous() if self.lda == self.K else _rows_ok(a)
-            if a.stride(0) != self.lda or a.data_ptr() % 16:
-                raise ValueError(f"PreparedStrips: activations need row stride {self.lda}, "
-                                 "16-byte aligned")
-            ptr = a.data_ptr()
+            if M != 1 or a.stride(1) != 1 or ptr & 15:  # one row may have any pitch
+                a = _packed_rows(a)
+                if a.stride(0) != self.lda and M > 1:
+                    raise ValueError(f"PreparedStrips: activations need row stride {self.lda}")
+                ptr = a.data_ptr()
         if out is None:
             ldc = self.N
             out = a.new_empty((M, ldc), dtype=self.out_dtype)

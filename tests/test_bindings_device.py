@@ -46,3 +46,25 @@ CASES = [
 def test_host_tensors_are_refused(name, call):
     with pytest.raises(ValueError, match=f"{name}: every tensor must be on one GPU"):
         call()
+
+
+ROW_FORMS = {
+    "second half of one row": lambda: _z(1, 512)[:, 256:], "odd pitch, one row": lambda: _z(1, 257)[:, :256],
+    "misaligned": lambda: _z(513)[1:].view(2, 256), "misaligned, one row": lambda: _z(257)[1:].view(1, 256),
+    "expanded": lambda: _z(256).expand(3, 256), "columns": lambda: _z(256, 3).t(),
+    "overlapping": lambda: _z(600).as_strided((3, 256), (4, 1)), "no rows": lambda: _z(0, 256),
+}
+
+
+@pytest.mark.parametrize("form", ROW_FORMS)
+def test_rows_for_the_kernels(form):
+    """Whatever form activations come in, the rows handed to a kernel have unit inner stride,
+    16-byte alignment and a pitch of at least their length -- also where torch calls the tensor
+    contiguous as it is (any base; one row of any pitch)."""
+    base = ROW_FORMS[form]()
+    x = torch.arange(base.numel(), dtype=torch.float32).view(base.shape)
+    if base.stride(0) >= base.shape[1] or base.shape[0] == 1:
+        base.copy_(x)
+    rows = _pk._rows_ok(base)
+    assert rows.stride(1) == 1 and rows.stride(0) >= 256 and rows.stride(0) % 4 == 0
+    assert rows.data_ptr() % 16 == 0 and torch.equal(rows, base)

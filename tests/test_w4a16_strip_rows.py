@@ -97,19 +97,23 @@ def test_quant_linear_batches(cuda, scheme, out_f):
 @pytest.mark.gpu
 @pytest.mark.parametrize("out_f", [1024, 17424])
 def test_quant_linear_batch_forms(cuda, out_f):
-    """Batches in forms other than contiguous, aligned rows: a misaligned base, a row pitch that
-    is a multiple of 16 bytes or not, transposed rows; each gives the contiguous copy's bits."""
+    """Decode rows and batches in forms other than contiguous, aligned rows: a misaligned base, a
+    row pitch that is a multiple of 16 bytes or not, the second half of wider rows, transposed
+    and expanded rows; each gives the contiguous copy's bits."""
     lin = torch.nn.Linear(256, out_f, device=cuda, dtype=torch.float16)
     q = quant_linear.QuantLinear.from_linear(lin, 128)
     rows = [M for M in (5, 9, 16, 32) if M > q.decode_rows and q._on_strips(M)]
     assert len(rows) >= 2
-    for M in rows:
+    for M in [1, 2, q.decode_rows] + rows:
         flat = torch.randn(M * 272 + 1, device=cuda).half()
         forms = (flat[1:M * 256 + 1].view(M, 256), flat[:M * 264].view(M, 264)[:, :256],
                  flat[:M * 264].view(M, 264)[:, 1:257], flat[:M * 257].view(M, 257)[:, :256],
-                 flat[:M * 256].view(256, M).t())
+                 flat[:M * 256].view(256, M).t(), flat[:256].expand(M, 256),
+                 torch.randn(M, 512, device=cuda).half()[:, 256:])
         for x in forms:
             assert torch.equal(q(x), q(x.clone(memory_format=torch.contiguous_format)))
+            xb = x.bfloat16() if x.stride(0) else x[:1].bfloat16().expand(M, 256)
+            assert torch.equal(q(xb), q(xb.clone(memory_format=torch.contiguous_format)))
         x = forms[0].view(1, M, 256)
         assert torch.equal(q(x)[0], q(forms[0].clone()))
 
