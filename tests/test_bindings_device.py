@@ -68,3 +68,18 @@ def test_rows_for_the_kernels(form):
     rows = _pk._rows_ok(base)
     assert rows.stride(1) == 1 and rows.stride(0) >= 256 and rows.stride(0) % 4 == 0
     assert rows.data_ptr() % 16 == 0 and torch.equal(rows, base)
+
+
+@pytest.mark.parametrize("q,v", [((1, 4, 1, 64), (2, 4, 256, 64)), ((2, 3, 1, 64), (2, 4, 256, 64)),
+                                 ((2, 8, 1, 64), (2, 4, 256, 64)), ((2, 4, 1, 32), (2, 4, 256, 64)),
+                                 ((2, 4, 1, 64), (2, 4, 128, 64)), ((2, 4, 1, 64), (1, 4, 256, 64)),
+                                 ((2, 4, 1, 64), (2, 4, 256, 32)), ((2, 4, 0, 64), (2, 4, 256, 64)),
+                                 ((2, 4, 32), (2, 4, 256, 64)), ((2, 4, 1, 1, 64), (2, 4, 256, 64)),
+                                 ((2, 4), (2, 4, 256, 64)), ((2, 4, 1, 64), (4, 256, 64))])
+def test_decode_shapes_are_checked(monkeypatch, q, v):
+    """q and v that do not fit k's (B, H, N, D) are refused before any library call: the kernel
+    would read past their ends, or answer for other heads than q's."""
+    monkeypatch.setattr(_pk, "_gpu_args", lambda *a: None)
+    monkeypatch.setattr(_pk, "stream_of", lambda t: pytest.fail("past the checks"))
+    with pytest.raises(ValueError, match="flash_decode: q"):
+        _pk.flash_decode(_z(*q, dtype=f16), _z(2, 4, 256, 64, dtype=f16), _z(*v, dtype=f16), 128, 0.125)

@@ -200,5 +200,6 @@ def test_query_forms(cuda):
         o = flash_decoding(q, k, v)
         assert o.shape == (2, 4, 1, 64) and o.is_contiguous()
         assert torch.equal(o, flash_decoding(q[:, :, :1].contiguous(), k, v))
+    assert torch.equal(flash_decoding(q, k[:, :, :256], v), flash_decoding(q, k[:, :, :256], v[:, :, :256]))
     with pytest.raises(IndexError):
         flash_decoding(wide[:, :, :0, :64], k, v)
