@@ -971,20 +971,29 @@ def flash_decode_launches(B: int, H: int, N: int, D: int, split: int) -> int:
 _fd_ws_bytes: dict[tuple[int, int, int, int, int], int] = {}
 
 
+def _decode_shapes(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+    """Raise unless q is (B, H, D) or (B, H, rows >= 1, D) and v (B, H, rows >= N, D) for k's
+    (B, H, N, D)."""
+    qs, vs = q.shape, v.shape
+    B, H, N, D = k.shape
+    if (len(qs) not in (3, 4) or (len(qs) == 4 and qs[2] < 1) or qs[:2] != (B, H) or qs[-1] != D
+            or len(vs) != 4 or vs[:2] != (B, H) or vs[2] < N or vs[3] != D):
+        raise ValueError(f"flash_decode: q {tuple(qs)}, k {tuple(k.shape)} and v {tuple(vs)} must be "
+                         "(B, H, D) or (B, H, rows, D), (B, H, N, D) and (B, H, N, D)")
+
+
 def flash_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, split: int,
                  sm_scale: float) -> torch.Tensor:
     """(B, H, D) fp32 single-query attention of q (B, H, D) over k, v (B, H, N, D), all fp16
     with unit stride along D (pk_flash_decode); (B, H, 1, D) for a 4-D q, its first row. Other
     shapes raise ``ValueError`` (rows of v beyond k's N are not read)."""
-    B, H, N, D = k.shape
-    sizes = q.shape
-    if (len(sizes) != 3 and (len(sizes) != 4 or sizes[2] < 1)
-            or sizes[0] != B or sizes[1] != H or sizes[-1] != D
-            or v.shape != k.shape and (v.dim() != 4 or v.shape[:2] != k.shape[:2]
-                                       or v.shape[2] < N or v.shape[3] != D)):
-        raise ValueError(f"flash_decode: q {tuple(sizes)}, k {tuple(k.shape)} and v {tuple(v.shape)} "
-                         "must be (B, H[, rows], D), (B, H, N, D) and (B, H, N, D)")
-    _gpu_args("flash_decode", q, k, v)
+    sizes = k.shape
+    B, H, N, D = sizes
+    if v.shape != sizes or (q.shape != (B, H, 1, D) and q.shape != (B, H, D)):
+        _decode_shapes(q, k, v)
+    dev = q.get_device()
+    if dev < 0 or k.get_device() != dev or v.get_device() != dev:
+        _gpu_args("flash_decode", q, k, v)
     sq, sk, sv = q.stride(), k.stride(), v.stride()
     if sq[-1] != 1 or (sq[0] | sq[1]) & 7 or q.data_ptr() & 15:
         q = q.contiguous()
