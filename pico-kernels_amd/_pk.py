@@ -321,15 +321,23 @@ def quantize_int4(w: torch.Tensor, scale: float) -> torch.Tensor:
     return q
 
 
+def _row_pitch(t: torch.Tensor) -> tuple[torch.Tensor, int]:
+    """A 2-D tensor whose rows have unit inner stride and do not overlap (else its contiguous
+    copy), and the pitch of its rows (their length where there is one, whatever its stride)."""
+    rows, cols = t.shape
+    if cols > 1 and t.stride(1) != 1 or rows > 1 and t.stride(0) < cols:
+        t = t.contiguous()
+    return t, t.stride(0) if rows > 1 else cols
+
+
 def pack_int4(q: torch.Tensor) -> torch.Tensor:
     _gpu_args("pack_int4", q)
     assert q.dim() == 2 and q.dtype == torch.int8
-    if q.stride(1) != 1:
-        q = q.contiguous()
+    q, ldq = _row_pitch(q)
     rows, cols = q.shape
     out = torch.empty((rows, cols // 2), dtype=torch.uint8, device=q.device)
-    _check(lib().pk_pack_int4(q.data_ptr(), rows, cols, max(q.stride(0), cols), out.data_ptr(),
-                              stream_of(q)), "pk_pack_int4")
+    _check(lib().pk_pack_int4(q.data_ptr(), rows, cols, ldq, out.data_ptr(), stream_of(q)),
+           "pk_pack_int4")
     return out
 
 
@@ -351,8 +359,7 @@ def quantize_group(w: torch.Tensor, bits: int, group_size: int | None, *, half_m
     """Group RTN along dim 0 of a 2-D (K, N) tensor. Returns (qweight, scales, fake)."""
     _gpu_args("quantize_group", w)
     assert w.dim() == 2
-    if w.stride(1) != 1:
-        w = w.contiguous()
+    w, ldw = _row_pitch(w)
     K, N = w.shape
     g = int(group_size) if group_size else 0
     ngroups = -(-K // g) if g else 1
@@ -361,7 +368,7 @@ def quantize_group(w: torch.Tensor, bits: int, group_size: int | None, *, half_m
     fdt = fake_dtype or w.dtype
     fake = torch.empty((K, N), dtype=fdt, device=w.device) if want_fake else None
     _check(lib().pk_quantize_group(
-        w.data_ptr(), pk_dtype(w.dtype), K, N, max(w.stride(0), N), int(bits), g, int(half_math),
+        w.data_ptr(), pk_dtype(w.dtype), K, N, ldw, int(bits), g, int(half_math),
         ptr(qweight), ptr(scales), pk_dtype(scale_dtype), ptr(fake), pk_dtype(fdt), stream_of(w)),
         "pk_quantize_group")
     return qweight, scales, fake

@@ -83,3 +83,43 @@ def test_decode_shapes_are_checked(monkeypatch, q, v):
     monkeypatch.setattr(_pk, "stream_of", lambda t: pytest.fail("past the checks"))
     with pytest.raises(ValueError, match="flash_decode: q"):
         _pk.flash_decode(_z(*q, dtype=f16), _z(2, 4, 256, 64, dtype=f16), _z(*v, dtype=f16), 128, 0.125)
+
+
+PITCHES = {  # (rows, columns, strides) and whether the kernel can read it in place
+    "expanded row": (5, 16, (0, 1), False), "expanded column": (5, 16, (1, 0), False),
+    "overlapping rows": (5, 16, (8, 1), False), "columns": (5, 16, (1, 5), False),
+    "contiguous": (5, 16, (16, 1), True), "wider rows": (5, 16, (24, 1), True),
+    "one row": (1, 16, (3, 1), True), "one expanded row": (1, 16, (0, 1), True),
+    "one column": (5, 1, (3, 7), True), "one expanded column": (5, 1, (0, 1), False),
+}
+
+
+@pytest.mark.parametrize("call,form", [("quantize_group", f) for f in PITCHES]
+                         + [("pack_int4", f) for f in PITCHES if PITCHES[f][1] % 2 == 0])
+def test_pitch_handed_to_the_kernel(monkeypatch, call, form):
+    """The row pitch a kernel is told is the tensor's own, or the tensor is copied: a pitch
+    below the row length rounded up to it would send the reads past the end."""
+    rows, cols, strides, in_place = PITCHES[form]
+    dt = torch.int8 if call == "pack_int4" else torch.float32
+    t = torch.zeros(200, dtype=dt).as_strided((rows, cols), strides)
+    seen = []
+
+    class Lib:
+        def pk_quantize_group(self, w, dtype, K, N, ld, *rest):
+            seen.append((w, K, N, ld))
+            return 0
+
+        def pk_pack_int4(self, q, K, N, ld, *rest):
+            seen.append((q, K, N, ld))
+            return 0
+
+    monkeypatch.setattr(_pk, "lib", Lib)
+    monkeypatch.setattr(_pk, "_gpu_args", lambda *a: None)
+    monkeypatch.setattr(_pk, "stream_of", lambda t: 0)
+    if call == "pack_int4":
+        _pk.pack_int4(t)
+    else:
+        _pk.quantize_group(t, 4, None, half_math=False, want_qweight=False, want_scales=False, want_fake=True)
+    (address, K, N, ld), = seen
+    assert (K, N) == (rows, cols) and (address == t.data_ptr()) == in_place
+    assert ld == (t.stride(0) if in_place and rows > 1 else cols)

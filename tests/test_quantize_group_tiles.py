@@ -79,3 +79,17 @@ def test_extremes(cuda):
             bad = qw.cpu().numpy().view(np.uint32)[:, 0] >> (4 * j) & 15
             r0 = (5 if j == 5 else 6) // g * g
             assert bad[5 if j == 5 else 6] == 0 and (bad[r0:r0 + g] == 0).all()
+
+
+@pytest.mark.parametrize("group", [64, None])
+def test_expanded_and_overlapping_weights(cuda, group):
+    """Weights whose rows share memory give the bits of their contiguous copy."""
+    g = torch.Generator().manual_seed(4)
+    row, col = torch.randn(72, generator=g).to(cuda), torch.randn(192, 1, generator=g).to(cuda)
+    for w in (row.expand(192, 72), col.expand(192, 72), row[:1].expand(192, 72),
+              torch.randn(4096, generator=g).to(cuda).as_strided((192, 72), (8, 1))):
+        outs = [_pk.quantize_group(x, 4, group, half_math=False, want_qweight=True, want_scales=True,
+                                   want_fake=True) for x in (w, w.contiguous())]
+        assert all(torch.equal(a, b) for a, b in zip(*outs))
+    codes = (row * 3).round().clamp(-8, 7).to(torch.int8).expand(192, 72)
+    assert torch.equal(_pk.pack_int4(codes), _pk.pack_int4(codes.contiguous()))
