@@ -68,10 +68,10 @@ const char* pk_last_error(void);
  * kernel posts a 32-bit value as message `seq` (a number the caller raises with every call
  * that posts to it; 0 is never used). pk_mailbox_create returns NULL on failure.
  * pk_mailbox_wait returns once message `seq` has come: the kernel that posts it has done its
- * work, not what was launched after it. It polls for 0.3 ms and then synchronises `stream`
- * (the stream of the posting call); PK_EHIP if the message has still not come. A mailbox may
- * be destroyed once no call that posts to it is pending. No counterpart in the reference
- * (torch's .item()). */
+ * work, not what was launched after it. It polls, after 0.3 ms with the core given up between
+ * polls; PK_EHIP if `stream` (the stream of the posting call) is done or has failed and the
+ * message has not come. A mailbox may be destroyed once no call that posts to it is pending.
+ * No counterpart in the reference (torch's .item()). */
 enum { PK_POST_COUNTER_BYTES = 2176 };
 void* pk_mailbox_create(void);
 void pk_mailbox_destroy(void* mailbox);

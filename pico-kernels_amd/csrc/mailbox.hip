@@ -8,6 +8,7 @@
 // kernel only, and what was launched behind it runs on meanwhile.
 #include "pk_internal.h"
 
+#include <sched.h>
 #include <time.h>
 
 using namespace pk;
@@ -38,22 +39,34 @@ extern "C" int pk_mailbox_wait(const void* box, uint32_t seq, uint32_t* value, v
     *value = (uint32_t)v;
     return true;
   };
-  // Poll for as long as a short queue takes; behind a longer one (or where a device's stores
-  // are not seen before its kernel ends) the stream's own wait does not burn the core.
-  constexpr int64_t kPollNs = 300 * 1000;
+  // Poll, for as long as a short queue takes without pause, behind a longer one with the core
+  // given up between polls: the stream's own wait would take in what was launched behind the
+  // post as well. A sleep lasts about 0.1 ms (the timer's slack), a small part of the wait by
+  // then. The stream is asked now and then, so that an error, or a message that never comes,
+  // ends the wait.
+  constexpr int64_t kSpinNs = 300 * 1000, kYieldNs = 3000 * 1000;
+  const timespec nap = {0, 50 * 1000};
   timespec t0, t;
   clock_gettime(CLOCK_MONOTONIC, &t0);
-  for (;;) {
+  for (unsigned turn = 1;; ++turn) {
     for (int i = 0; i < 64; ++i) {
       if (arrived()) return PK_OK;
       __builtin_ia32_pause();
     }
     clock_gettime(CLOCK_MONOTONIC, &t);
-    if ((t.tv_sec - t0.tv_sec) * 1000000000ll + (t.tv_nsec - t0.tv_nsec) > kPollNs) break;
+    const int64_t waited = (t.tv_sec - t0.tv_sec) * 1000000000ll + (t.tv_nsec - t0.tv_nsec);
+    if (waited <= kSpinNs) continue;
+    if (waited <= kYieldNs) sched_yield();
+    else nanosleep(&nap, nullptr);
+    if (turn % 16 != 0) continue;
+    const hipError_t e = hipStreamQuery((hipStream_t)stream);
+    if (e == hipErrorNotReady) {
+      (void)hipGetLastError();  // no error: the next launch must not find it
+      continue;
+    }
+    if (e != hipSuccess) return hip_status(e, "pk_mailbox_wait: hipStreamQuery");
+    if (arrived()) return PK_OK;
+    set_error("pk_mailbox_wait: the stream is done and message %u has not come", seq);
+    return PK_EHIP;
   }
-  const hipError_t e = hipStreamSynchronize((hipStream_t)stream);
-  if (e != hipSuccess) return hip_status(e, "pk_mailbox_wait: hipStreamSynchronize");
-  if (arrived()) return PK_OK;
-  set_error("pk_mailbox_wait: the stream is done and message %u has not come", seq);
-  return PK_EHIP;
 }

@@ -71,6 +71,33 @@ def test_threads_and_streams(cuda):
     assert not wrong and not any(t.is_alive() for t in threads)
 
 
+@pytest.mark.parametrize("ahead", [0, 1, 8])
+def test_waits_for_its_own_pass_only(cuda, ahead):
+    """Whatever is queued before the pass (8192^3 products of about a millisecond each), the answer
+    comes when the pass is done, with what was launched behind it still under way."""
+    a = torch.ones(8192, 8192, device=cuda, dtype=torch.float16)
+    out = torch.empty_like(a)
+    x = torch.ones(8, 4096, device=cuda, dtype=torch.bfloat16)
+    torch.mm(a, a, out=out)
+    _run(x)
+    for value in (1.0, 1e5):
+        x[7, 4095] = value
+        torch.cuda.synchronize()
+        for _ in range(ahead):
+            torch.mm(a, a, out=out)
+        try:
+            with _pk.checked_activations(x, None, 1.0, "t") as y:
+                for _ in range(60):
+                    torch.mm(a, a, out=out)
+            raised = False
+        except ValueError:
+            raised = True  # (the message's maximum synchronises)
+        else:
+            assert not torch.cuda.current_stream().query()
+        torch.cuda.synchronize()
+        assert raised == (value > 65504) and torch.equal(y, x.half())
+
+
 def test_capture_runs_the_plain_pass(cuda):
     x = torch.full((4, 256), 1e5, device=cuda, dtype=torch.bfloat16)
     _run(torch.ones_like(x))
