@@ -123,7 +123,8 @@ int pk_unpack_int4(const uint8_t* packed, int64_t rows, int64_t cols, int8_t* q,
  *   qweight   (K, N/8) int32: 4-bit codes, byte-identical to pack_int4_n (bits must be 4,
  *             N % 8 == 0)
  *   scales    (ceil(K/G), N) in `scale_dtype` (PK_F16 or PK_F32), RNE-rounded from s
- *   fake      (K, N) in `fake_dtype`: T(q * s), the tensor rtn_layer returns
+ *   fake      (K, N) in `fake_dtype`: T(q * s), the tensor rtn_layer returns; may be w itself
+ *             (w's dtype, ldw == N), else the buffers must not overlap
  * half_math != 0 reproduces quantize_col applied directly to an fp16 tensor (every op
  * rounded to fp16, the 1e-12 floor becoming 0); it requires w_dtype == PK_F16.
  * Replaces quantize.rtn_layer / quantize.quantize_col (quantize.py:42-68) and is the

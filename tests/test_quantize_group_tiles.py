@@ -93,3 +93,20 @@ def test_expanded_and_overlapping_weights(cuda, group):
         assert all(torch.equal(a, b) for a, b in zip(*outs))
     codes = (row * 3).round().clamp(-8, 7).to(torch.int8).expand(192, 72)
     assert torch.equal(_pk.pack_int4(codes), _pk.pack_int4(codes.contiguous()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("K,N,group,half_math", [(130, 264, 128, 0), (700, 72, 0, 0), (1030, 40, 513, 0),
+                                                 (96, 13, 32, 0), (333, 8, 0, 1)])
+def test_in_place(cuda, dtype, K, N, group, half_math):
+    """Values written over the weights: those of a separate buffer, also in the rows on and beside a
+    rounding tie, which are read a second time."""
+    w = _weights(K, N, dtype, K + N).to(cuda)
+    if half_math and dtype == torch.float32:
+        half_math = 0
+    want = _pk.quantize_group(w, 4, group, half_math=bool(half_math), want_qweight=False,
+                              want_scales=False, want_fake=True)[2]
+    dt = _pk.pk_dtype(dtype)
+    rc = _pk.lib().pk_quantize_group(w.data_ptr(), dt, K, N, N, 4, group, half_math, None, None, dt,
+                                     w.data_ptr(), dt, _pk.stream_of(w))
+    assert rc == _pk.PK_OK and torch.equal(w, want)
