@@ -371,6 +371,10 @@ int pk_gemm_f16(const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                 int64_t ldc, int M, int N, int K, int split_k, void* workspace,
                 size_t workspace_bytes, void* stream);
 
+/* Rows (64 or 128) of the 256-column tiles that a pk_gemm_f16 / _bf16 call with 16-byte aligned operands
+ * is planned on; 0 where another kernel runs it; PK_EINVAL for a call no kernel takes. */
+int pk_gemm_f16_tile_rows(int M, int N, int K, int split_k);
+
 /* pk_gemm_f16 with bf16 A and B (bf16 MFMA, fp32 accumulate); the same constraints and
  * workspace (pk_gemm_f16_workspace_bytes). Replaces gemm.triton_gemm (gemm.py:103-128) for
  * bf16 and gemm_splitk.triton_gemm_splitk (gemm_splitk.py:67-80) with bf16 inputs; the

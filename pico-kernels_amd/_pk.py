@@ -91,6 +91,7 @@ _SIGNATURES = {
                                       _i32, _vp]),
     "pk_splitk_reduce": (_i32, [_vp, _i32, _i32, _i32, _f32, _vp, _i32, _i64, _vp]),
     "pk_gemm_f16_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "pk_gemm_f16_tile_rows": (_i32, [_i32, _i32, _i32, _i32]),
     "pk_gemm_f16": (_i32, [_vp, _i64, _vp, _i64, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp,
                            _sz, _vp]),
     "pk_gemm_bf16": (_i32, [_vp, _i64, _vp, _i64, _vp, _i32, _i64, _i32, _i32, _i32, _i32, _vp,

@@ -6,7 +6,7 @@
 // for 128 bytes per clock at full matrix rate, beside the B tile's ds_writes, byte permutes
 // and registers. Here nothing passes through registers on its way in, and a wave's block is
 // 128 x 64:
-//  * BM x 256 workgroup tiles (BM = 128, or 64 where that takes less time: dense_tr_launch), k-tiles
+//  * BM x 256 workgroup tiles (BM = 128, or 64 where that takes less time: dense_tr_rows), k-tiles
 //    of 32, eight waves. Wave w owns columns 64 (w % 4) .. +63 of all the tile's rows and the k half
 //    h = w / 4 of every k-tile: waves w and w + 4 share a SIMD, compute the same block over
 //    different k and add their accumulators once, at the end. LDS serves 96 bytes per clock at
@@ -299,6 +299,15 @@ bool dense_tr_ok(int M, int N, int K, int split, int64_t lda, const void* b, int
   return (int64_t)M * lda * 2 < (1ll << 31) && (int64_t)K * ldb * 2 < (1ll << 31);
 }
 
+// 64-row tiles where as many rounds of the 256 CUs do (which is one round): 1024 x 4096 x 4096, 128 or
+// 256 tiles: 51.7 against 42.7 us. A round of them takes 0.7 to 0.85 of one of 128 rows, so one
+// more round is never made good: bf16 3840 x 2048 x 1600, 240 tiles of 128 rows 28.6 us, 480 of 64 rows
+// 44; 3072 x 4096 x 2048, 384 or 768 tiles: 62 against 68.
+int dense_tr_rows(int M, int N, int split) {
+  auto rounds = [&](int rows) { return cdiv(cdiv(M, rows) * (N / 256) * split, 256); };
+  return rounds(64) == rounds(128) ? 64 : 128;
+}
+
 int dense_tr_launch(bool bf16, const void* a, int64_t lda, const void* b, int64_t ldb, void* c,
                     int c_dtype, int64_t ldc, int M, int N, int K, int split, float* partials,
                     hipStream_t s) {
@@ -315,11 +324,7 @@ int dense_tr_launch(bool bf16, const void* a, int64_t lda, const void* b, int64_
   p.K = K;
   p.kt_slice = K / split / 32;
   p.tiles_n = N / 256;
-  // 64-row tiles where they take less time: a round of them takes about 0.6 of one of 128 rows
-  // (bf16 3840 x 2048 x 1600, 240 tiles of 128 rows: 28.6 us, with 480 of 64 rows 44; 1024 x 4096 x
-  // 4096, 128 or 256 tiles: 51.7 against 42.7 us)
-  auto rounds = [&](int rows) { return cdiv(cdiv(M, rows) * p.tiles_n * split, 256); };
-  const int bm = 6 * rounds(64) < 10 * rounds(128) ? 64 : 128;
+  const int bm = dense_tr_rows(M, N, split);
   p.tiles_m = (int)cdiv(M, bm);
   const dim3 grid(p.tiles_m * p.tiles_n, split);
   if (bf16 && bm == 128) gemm_dense_tr_kernel<true, 128><<<grid, 512, 0, s>>>(p);

@@ -405,6 +405,14 @@ extern "C" size_t pk_gemm_f16_workspace_bytes(int M, int N, int K, int split_k) 
   return gemm_workspace_bytes(pl, M, N);
 }
 
+extern "C" int pk_gemm_f16_tile_rows(int M, int N, int K, int split_k) {
+  GemmPlan pl;
+  PK_REQUIRE(M >= 1 && N >= 1 && K >= 1 && gemm_plan(M, N, K, K, false, split_k, &pl),
+             "pk_gemm_f16_tile_rows: no kernel for M=%d N=%d K=%d split_k=%d", M, N, K, split_k);
+  if (!dense_tr_ok(M, N, K, pl.split, K, nullptr, N, N, PK_F32, nullptr)) return 0;
+  return dense_tr_rows(M, N, pl.split);
+}
+
 // Dense C = A @ B for fp16 (bmode 0) or bf16 (bmode 2) operands.
 static int gemm_dense(const char* name, int bmode, const void* a, int64_t lda, const void* b,
                       int64_t ldb, void* c, int c_dtype, int64_t ldc, int M, int N, int K,

@@ -9,13 +9,11 @@ import torch
 
 import _pk
 
-pytestmark = pytest.mark.gpu
-
-
 def _rel(y, ref):
     return ((y.double() - ref).norm() / ref.norm()).item()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("M,K,N,split", [
     (64, 32, 256, 1), (65, 64, 256, 1), (128, 96, 512, 1), (200, 160, 256, 1), (256, 192, 256, 1),
@@ -32,3 +30,15 @@ def test_against_fp64(cuda, dtype, M, K, N, split):
     assert torch.equal(y, _pk.gemm_dense(a, b, torch.float32, split))
     for dt in (torch.float16, torch.bfloat16):
         assert torch.equal(_pk.gemm_dense(a, b, dt, split), y.to(dt))
+
+
+@pytest.mark.parametrize("M,N,K,split,rows", [
+    (1024, 4096, 4096, 1, 64), (2048, 2048, 512, 1, 64), (2048, 4096, 4096, 1, 128),  # 256, 256 and 512 of 64
+    (3072, 4096, 2048, 1, 128), (3072, 3072, 512, 1, 128), (4096, 3072, 1024, 1, 128),  # three rounds for two
+    (4096, 4096, 4096, 1, 128), (512, 512, 8192, 4, 64), (1024, 1024, 8192, 8, 128), (64, 65536 + 256, 32, 1, 64),
+    (48, 256, 64, 1, 0), (256, 264, 64, 1, 0)])
+def test_tile_rows(M, N, K, split, rows):
+    """64-row tiles only where they need no round more than 128-row ones: three rounds of them for
+    two took 1.06 to 1.2 times as long."""
+    assert _pk.lib().pk_gemm_f16_tile_rows(M, N, K, split) == rows
+    assert _pk.lib().pk_gemm_f16_tile_rows(M, N, K + 1, split) < 0
