@@ -293,6 +293,15 @@ bool dense_tr_ok(int M, int N, int K, int split, int64_t lda, const void* b, int
                  int64_t ldc, int c_dtype, const void* c) {
   const int es = c_dtype == PK_F32 ? 4 : 2;
   if (N % 256 || K % (32 * split) || M < 64) return false;
+  // A whole round of workgroups or more with slices of at most 1024 k is left to gemm_v3_f16_kernel
+  // (slices of whole 64s). This kernel runs into the card's power limit there: its time depends on
+  // what ran before and on the operands (fp16 2048 x 4096 x 512, both kernels in turn: 16.5 against
+  // 17.6 us after a long run, 21 to 24 against 18.1 in bursts of 5 to 100, 14.5 against 15.8 on zeros), and
+  // bursts take, old / new us: fp16 2048 x 4096 x 384 16.7 / 20.6, 3072 x 4096 x 512 29.2 / 32.5, 4096^2 x 768
+  // 42.4 / 46.0, 2048 x 4096 x 1024 26.0 / 28.1; x 1536 34.3 / 30.7, 4096^2 x 1536 65.5 / 59.7. Fewer tiles have no
+  // such K: 2048 x 3072 x 512 16.6 / 14.5, 1024 x 4096 x 256 11.8 / 8.5.
+  const int64_t tiles = cdiv(M, 128) * (N / 256) * split;
+  if (tiles >= 256 && K / split <= 1024 && K / split % 64 == 0) return false;
   if (ldb % 8 || (reinterpret_cast<uintptr_t>(b) & 15)) return false;
   if (split == 1 && ((ldc * es) % 16 || (reinterpret_cast<uintptr_t>(c) & 15))) return false;
   // 32-bit buffer offsets

@@ -180,8 +180,9 @@ int v2_f16_launch(int bm, int bmode, const void* a, int64_t lda, const void* b, 
                   int M, int N, int K, int split, void* workspace, hipStream_t s,
                   bool partials_only);
 // Dense fp16 / bf16 GEMM on 128 x 256 or 64 x 256 tiles, B read by transposing LDS reads
-// (gemm_dense_tr.hip): M >= 64, N % 256 == 0, K % (32 * split) == 0; split > 1 writes fp32 partial
-// planes to `partials` and reduces them. dense_tr_rows: the rows of its tiles.
+// (gemm_dense_tr.hip): M >= 64, N % 256 == 0, K % (32 * split) == 0 (dense_tr_ok says where it is the
+// faster kernel too); split > 1 writes fp32 partial planes to `partials` and reduces them.
+// dense_tr_rows: the rows of its tiles.
 bool dense_tr_ok(int M, int N, int K, int split, int64_t lda, const void* b, int64_t ldb,
                  int64_t ldc, int c_dtype, const void* c);
 int dense_tr_rows(int M, int N, int split);
