@@ -389,8 +389,8 @@ def absmax_cast_e4m3(x: torch.Tensor) -> tuple[torch.Tensor, float]:
     launched at once, and the host waits for the maximum alone."""
     _gpu_args("cast_e4m3", x)
     if torch.cuda.is_current_stream_capturing():
-        m = absmax(x).item()  # raises: no host wait while a graph is captured
-        return cast_e4m3(x, 448.0 / m), m
+        raise RuntimeError("absmax_cast_e4m3: the maximum cannot be handed to the host while a graph "
+                           "is captured")
     x = x.contiguous()
     out = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device)
     L = lib()
@@ -448,23 +448,6 @@ def w4a16_launches(M: int, N: int, K: int, group_size: int, split_k: int) -> int
     return n
 
 
-FP16_MAX = 65504.0
-
-
-def check_fp16_range(x: torch.Tensor, what: str, converted: torch.Tensor | None = None) -> None:
-    """Raise ``ValueError`` when a finite element of ``x`` (bf16 / fp32 activations the W4A16
-    kernels take as fp16) lies beyond fp16's largest finite value 65504, where the fp16 cast
-    would turn it into an infinity -- or, given ``converted`` (the fp16 tensor made from
-    ``x``), when a finite element of ``x`` became infinite in it. One device reduction and a
-    synchronisation; skipped while the stream is being captured into a graph (no
-    synchronisation is allowed there)."""
-    if x.dtype == torch.float16 or (x.is_cuda and torch.cuda.is_current_stream_capturing()):
-        return
-    bad = torch.isinf(converted) if converted is not None else x.abs() > FP16_MAX
-    if bool((bad & torch.isfinite(x)).any()):
-        _raise_fp16_range(x, what)
-
-
 def _raise_fp16_range(x: torch.Tensor, what: str) -> None:
     big = x[torch.isfinite(x)].abs().max().item()
     raise ValueError(f"{what}: {x.dtype} activations up to |x| = {big:g} exceed fp16's range "
@@ -472,10 +455,11 @@ def _raise_fp16_range(x: torch.Tensor, what: str) -> None:
 
 
 class checked_activations:
-    """``w4a16_prep_activations`` with the range check of ``check_fp16_range`` in the same pass
+    """``w4a16_prep_activations`` with a range check in the same pass
     (``pk_w4a16_prep_checked``): ``out`` is the fp16 tensor, for launches made inside the
     ``with`` block; leaving the block waits for the check's answer and raises ``ValueError`` if
-    a finite element became infinite. Under graph capture (no host wait is possible) and for
+    a finite element (of the bf16 / fp32 activations the W4A16 kernels take as fp16) became
+    infinite, being beyond 65504 after the scales. Under graph capture (no host wait is possible) and for
     inputs with nothing to check, the plain pass."""
 
     def __init__(self, x: torch.Tensor, in_scale: torch.Tensor | None, mul: float, what: str):
@@ -778,7 +762,8 @@ class PreparedStrips:
         return out
 
     def timed(self, a: torch.Tensor, out: torch.Tensor, start=None, stop=None) -> None:
-        """The call above (activations as the prepared stride wants them, output given), with
+        """The decode kernel's launch for 1..8 rows -- the call above below ``rows_from`` -- on
+        activations as the prepared stride wants them and a given output, with
         ``torch.cuda.Event`` ``start`` recorded as its kernel starts and ``stop`` as it ends, by
         the dispatch itself (``pk_w4a16_strips_run_events``). Each event is recorded once on
         the current stream first if it has no HIP event yet."""

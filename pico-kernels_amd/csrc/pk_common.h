@@ -174,54 +174,10 @@ __device__ __forceinline__ void with_dtype(int dtype, F f) {
   else f(pk_int_c<PK_BF16>{});
 }
 
-// OCP FP8 E4M3 ("e4m3fn": no infinities, S.1111.111 is NaN, max finite 448).
-// Round-to-nearest-even, NOT saturating: any magnitude that rounds above 448 (that is,
-// anything above 464, the tie point between 448 and the missing 480) and any Inf/NaN input
-// becomes NaN (0x7f | sign). Written from the format definition:
-//   normal:    (-1)^s * 2^(e-7) * (1 + m/8),   e in 1..15 (e=15,m=7 reserved for NaN)
-//   subnormal: (-1)^s * 2^-6 * (m/8)
-__host__ __device__ __forceinline__ uint8_t e4m3_from_f32(float f) {
-  uint32_t u = __builtin_bit_cast(uint32_t, f);
-  uint8_t sign = (uint8_t)((u >> 24) & 0x80u);
-  uint32_t a = u & 0x7fffffffu;
-  if (a > 0x43e80000u) return sign | 0x7fu;           // > 464.0, Inf or NaN
-  if (a < 0x3c800000u) {                              // below 2^-6: subnormal grid of 2^-9
-    float mag = __builtin_bit_cast(float, a) * 512.0f;  // exact (power-of-two scaling)
-    return sign | (uint8_t)__builtin_rintf(mag);      // 0..8; 8 is the smallest normal
-  }
-  // Normal range [2^-6, 464]: keep 3 mantissa bits with round-to-nearest-even. Adding
-  // (half ulp - 1) plus the kept LSB then truncating is RNE; a mantissa carry correctly
-  // bumps the exponent field.
-  uint32_t r = (a + 0x7ffffu + ((a >> 20) & 1u)) >> 20;  // = (f32 exp << 3) | mant3
-  return sign | (uint8_t)(r - ((127u - 7u) << 3));
-}
-
-__host__ __device__ __forceinline__ float e4m3_to_f32(uint8_t v) {
-  uint32_t s = (uint32_t)(v & 0x80u) << 24;
-  uint32_t e = (v >> 3) & 15u, m = v & 7u;
-  if (e == 15u && m == 7u) return __builtin_bit_cast(float, s | 0x7fc00000u);
-  float mag;
-  if (e == 0) mag = (float)m * (1.0f / 512.0f);
-  else mag = __builtin_bit_cast(float, ((e + 120u) << 23) | (m << 20));
-  return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, mag) | s);
-}
-
-// NaN-propagating max of non-negative values (torch's max propagates NaN).
-__device__ __forceinline__ float nanmax(float a, float b) {
-  if (a != a) return a;
-  if (b != b) return b;
-  return a > b ? a : b;
-}
-
 // Clamp that propagates NaN the way torch.clamp does.
 __device__ __forceinline__ float clamp_nan(float x, float lo, float hi) {
   return x < lo ? lo : (x > hi ? hi : x);
 }
-
-// ---------------------------------------------------------------------------------------
-// Wave-level helpers (wave64).
-// ---------------------------------------------------------------------------------------
-__device__ __forceinline__ float wave_shfl_xor(float v, int mask) { return __shfl_xor(v, mask, 64); }
 
 // ---------------------------------------------------------------------------------------
 // Split-K reduction inside one XCD's L2.

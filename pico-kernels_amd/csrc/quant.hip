@@ -503,7 +503,13 @@ __global__ __launch_bounds__(kQgLongThreads) void quantize_group_long_kernel(QgP
 // stores (the rest, and misaligned operands, element by element). Measured on MI355X, 1000 x 4096 bf16: 8.0 ->
 // 5.6 us; 4096 x 6144 bf16 33 -> 18.9 us (2-byte loads and branches before).
 // ---------------------------------------------------------------------------------------
-// e4m3_from_f32 without branches (the same bits).
+// OCP FP8 E4M3 ("e4m3fn": no infinities, S.1111.111 is NaN, max finite 448), round to nearest even,
+// not saturating: what rounds above 448 (anything above 464, the tie with the missing 480), Inf
+// and NaN become NaN (0x7f | sign). From the format's definition, without branches:
+//   normal:    (-1)^s * 2^(e-7) * (1 + m/8), e in 1..15 (e = 15, m = 7 reserved for NaN): half an ulp
+//              less one plus the kept lowest bit added, then truncated; a carry out of the
+//              mantissa raises the exponent
+//   subnormal: (-1)^s * 2^-6 * (m/8): whole multiples of 2^-9 (8 of them the smallest normal)
 __device__ __forceinline__ uint32_t e4m3_select(float f) {
   const uint32_t u = __builtin_bit_cast(uint32_t, f), a = u & 0x7fffffffu;
   const uint32_t sub = (uint32_t)__builtin_rintf(__builtin_bit_cast(float, a) * 512.0f);

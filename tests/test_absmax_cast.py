@@ -61,3 +61,19 @@ def test_every_16_bit_value(cuda, dtype):
             want = oracle.e4m3_from_f32((x.float() * np.float32(scale)).to(dtype).float().numpy())
         nan = x.isnan().numpy()  # torch drops a NaN's sign where it rounds to bf16
         assert np.array_equal(out[~nan], want[~nan]) and (out[nan] & 0x7f == 0x7f).all()
+
+
+def test_refused_under_capture(cuda):
+    """The scale goes to the host, so a capture cannot hold the call; the capture goes on."""
+    x = torch.full((64,), 3.0, device=cuda)
+    gemm_fp8.quantize(x)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="captured"):
+            gemm_fp8.quantize(x)
+        y = _pk.cast_e4m3(x, 2.0)
+    for v in (1.0, 5.0):
+        x.fill_(v)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool((y.float() == 2 * v).all())

@@ -11,20 +11,30 @@ import torch
 import _pk
 
 
-def test_range_check_host_logic():
-    ok = torch.tensor([65504.0, -65504.0, 1e-30, float("inf"), float("nan")])
-    _pk.check_fp16_range(ok, "t")                       # the edge itself, non-finite inputs
-    _pk.check_fp16_range(ok.to(torch.bfloat16), "t")
+def _check(values, dtype=torch.float32, scales=None):
+    x = torch.zeros(1, 8)
+    x[0, :len(values)] = torch.tensor(values)
+    with _pk.checked_activations(x.to(dtype).cuda(), scales, 1.0, "t"):
+        pass
+
+
+@pytest.mark.gpu
+def test_range_check(cuda):
+    ok = [65504.0, -65504.0, 1e-30, float("inf"), float("nan")]
+    _check(ok)                                          # the edge itself, non-finite inputs
+    _check([1.0] + ok[2:], torch.bfloat16)              # (65504 is no bf16: 65536 is beyond)
     with pytest.raises(ValueError, match="exceed fp16's range"):
-        _pk.check_fp16_range(torch.tensor([1.0, 70000.0]), "t")
+        _check([1.0, 70000.0])
     with pytest.raises(ValueError):
-        _pk.check_fp16_range(torch.tensor([-1e5], dtype=torch.bfloat16), "t")
-    # given the converted tensor, only finite inputs that turned infinite count
-    x = torch.tensor([1e5, 2.0])
-    _pk.check_fp16_range(x, "t", torch.tensor([1.0, 2.0], dtype=torch.float16))
+        _check([-1e5], torch.bfloat16)
+    # after the scales, only finite inputs that turned infinite count
+    scales = torch.full((8,), 1e-5, device=cuda)
+    _check([1e5, 2.0], scales=scales)
     with pytest.raises(ValueError):
-        _pk.check_fp16_range(x, "t", x.half())
-    _pk.check_fp16_range(torch.tensor([7e4]).half(), "t")  # already fp16: nothing to check
+        _check([1e5, 2.0])
+    with pytest.raises(ValueError):
+        _check([2.0], scales=scales * 1e10)
+    _check([7e4], torch.float16)                        # already fp16: nothing to check
 
 
 @pytest.mark.gpu
