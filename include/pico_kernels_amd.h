@@ -11,7 +11,7 @@
  * Conventions
  *  - Plain pointers and sizes only. Device pointers are HIP device memory; `stream` is a
  *    hipStream_t passed as void* (NULL = the default stream). All launches are asynchronous
- *    on `stream`; nothing here synchronises the device.
+ *    on `stream`; nothing here synchronises the device, and only pk_mailbox_wait waits.
  *  - The library never allocates device memory. Entry points that need scratch space take
  *    a caller-owned `workspace` whose size is given by the matching *_workspace_bytes().
  *    The workspace of pk_w4a16_gemm / pk_gemm_f16 starts with 64 KiB of split-K arrival
