@@ -600,6 +600,8 @@ def w4a16_gemm_strips(a: torch.Tensor, qstrips: torch.Tensor, sstrips: torch.Ten
     M, K = a.shape
     N = qstrips.shape[1] * 8
     a = _rows_ok(a)
+    if M * a.stride(0) >= 1 << 30:  # the kernels address less than 2 GiB of activations
+        a = _packed_rows(a)
     if out is None:
         out = torch.empty((M, N), dtype=out_dtype, device=a.device)
     g = int(group_size) if sstrips is not None else 0

@@ -123,3 +123,26 @@ def test_pitch_handed_to_the_kernel(monkeypatch, call, form):
     (address, K, N, ld), = seen
     assert (K, N) == (rows, cols) and (address == t.data_ptr()) == in_place
     assert ld == (t.stride(0) if in_place and rows > 1 else cols)
+
+
+@pytest.mark.parametrize("rows", [1, 9, 64])
+def test_rows_far_apart(monkeypatch, rows):
+    """Rows that span 2 GiB or more, as the kernels on the row layout take them, are packed for the
+    strip kernels, whose offsets have 32 bits."""
+    seen = []
+
+    class Calls:
+        def pk_w4a16_gemm_strips_rows(self, a, lda, *rest):
+            seen.append(lda)
+            return 0
+
+        pk_w4a16_gemm_strips = pk_w4a16_gemm_strips_rows
+
+    monkeypatch.setattr(_pk, "_calls", Calls())
+    monkeypatch.setattr(_pk, "_gpu_args", lambda *a: None)
+    monkeypatch.setattr(_pk, "stream_of", lambda t: 0)
+    weights = torch.empty(256, 32, dtype=i32, device="meta")
+    for pitch in ((1 << 30) // rows // 8 * 8 - 8, (1 << 30) // rows // 8 * 8 + 8):
+        a = torch.empty(rows * pitch, dtype=f16, device="meta").view(rows, pitch)[:, :256]
+        _pk.w4a16_gemm_strips(a, weights, None, 0, 1.0, f16, rows=rows > 8)
+        assert rows * seen[-1] < 1 << 30 and seen[-1] == (pitch if rows * pitch < 1 << 30 else 256)
