@@ -1007,7 +1007,7 @@ def flash_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, split: int,
         if len(_fd_ws_bytes) > 4096:
             _fd_ws_bytes.clear()
         nbytes = _fd_ws_bytes[key] = lib().pk_flash_decode_workspace_bytes(B, H, N, D, split)
-    stream = stream_of(q)
+    stream = torch._C._cuda_getCurrentRawStream(dev)
     ws = workspace(q.device, nbytes, stream)  # zero-filled counters, shared with the GEMMs
     rc = (_calls or calls()).pk_flash_decode(
         q.data_ptr(), sq[0], sq[1], k.data_ptr(), sk[0], sk[1], sk[2], v.data_ptr(), sv[0], sv[1],
