@@ -644,9 +644,10 @@ def strip_batch(M: int, K: int, N: int, group_size: int, blocks: bool) -> bool:
       above 32 rows, packed-B GEMM planned: it fills the chip, unless K leaves it one slice.
         8064 x 9216 g M = 64 24.0 / 41.3, 7040 x 5120 g M = 51 17.2 / 20.1; one slice: 13952 x 6144 g
         M = 33 101 / 32.8, 9856 x 12032 g M = 64 70.3 / 50.1, but 3712 x 11520 t M = 54 21.7 / 25.5
-      above 32 rows, register-dequant kernel planned: 4096 x 14352 M = 48 g 30.8 / 24.8, t 24.2 / 25.8;
-        3072 x 8864 g M = 41 17.6 / 20.3 (277 workgroups); 11520 x 5872 t M = 33 25.1 / 28.4; few strips:
-        13312 x 1920 g M = 48 17.2 / 26.1, 9600 x 3280 t M = 36 18.6 / 20.2
+      above 32 rows, register-dequant kernel planned: 4096 x 14352 M = 48 g 30.8 / 24.8 (452 of its
+        workgroups), t 24.2 / 25.8 (226); 2048 x 12928 g M = 33 14.8 / 16.0 (202); 3072 x 8864 g M = 41 17.6
+        / 20.3 (277 batch workgroups); 11520 x 5872 t M = 33 25.1 / 28.4; few strips: 13312 x 1920 g M = 48
+        17.2 / 26.1, 14336 x 3408 t M = 47 22.3 / 28.6
       up to 32 rows: 4096 x 14352 M = 32 g 20.9 / 14.2; few strips of a long K: 13312 x 1920 g M = 31
         14.0 / 16.8, 8192 x 1536 g M = 11 7.7 / 8.4; 129 to 160 workgroups of four strips against a few
         slices: 6144 x 8960 g M = 26 16.2 / 17.3; just beyond 1024 strips: 7168 x 17408 g M = 9 22.0 /
@@ -659,32 +660,43 @@ def strip_batch(M: int, K: int, N: int, group_size: int, blocks: bool) -> bool:
         return False
     kernel, split = w4a16_plan(M, N, K, group_size, 0)
     strips, slice_rows = N // 16, K // split
-    whole = group_size >= 128  # groups of whole 128-row blocks
+    plan_wgs = -(-N // 128) * split  # of the register-dequant kernel
+    whole, short = group_size >= 128, 0 < group_size < 128  # groups of whole 128-row blocks
     if M > 32:
         if kernel == PLAN_PACKED_B:
             if split == 1:
                 return strips <= (1024 if whole else 512)
             return whole and split <= 3 and strips <= 512
-        if strips <= (128 if whole else 208) and K >= 4096 and split <= 16:
-            return False
         if strips <= 128:
-            return K <= 6144 or slice_rows < (256 if 0 < group_size < 128 else 384)
+            return not (K >= 4096 and split <= 16) and (K <= 6144 or slice_rows < (256 if short else 384))
+        eight = slice_rows % 256 == 0  # waves of its workgroups, one on a CU (else four, two)
         if strips <= 512:
-            return whole or split >= 8 or K <= 4096
-        if slice_rows <= 256 and (whole or group_size == 0):
+            if whole:  # 8192 x 3696 M = 38 16.7 / 17.8 (232 workgroups)
+                return not (K > 7168 and strips > 208 and eight and plan_wgs <= 256)
+            return K <= 9408 or plan_wgs > (256 if eight else 448)
+        if short:
+            return split >= 9 if strips > 1024 else K <= 512
+        if slice_rows <= 320:
             return True
-        if strips <= 1024:
-            return whole and (strips > 576 or K <= 2048) or K <= 512
-        return split >= (3 if whole else 9)
-    if strips <= (128 if K < 12288 else 192):
+        if strips > 1024:
+            return split >= (3 if whole else 9)
+        if whole:
+            return plan_wgs > 256 and (strips > 656 or split % 2 == 1 or not 384 < plan_wgs <= 512)
+        if eight:
+            return strips > 656 and (256 < plan_wgs <= 352 or plan_wgs > 512)
+        return plan_wgs > 512 and strips > (656 if slice_rows < 1152 else 800)
+    if strips <= (192 if K >= 12288 and blocks else 128):
         if slice_rows < 512 or K < (8192 if M <= 16 else 6400):
             return True
-        return not (blocks or M <= 16 or K >= 12288 or 0 < group_size < 128)
+        return not (blocks or short or M <= 16 or K >= 12288)
     if strips <= 1024:
         return strips <= 512 or strips > 640 or K < 6144 or split > 3
     if strips <= 1408:
-        return ((split >= 9 and slice_rows <= 512) or (split == 2 and K >= 3072)
-                or (not blocks and whole and split != 3))
+        if slice_rows <= 384 and (M > 16 or plan_wgs > 1400) or split >= 9 and slice_rows <= 512:
+            return True
+        if split == 2:
+            return K >= 3072 or M > 16 or not blocks
+        return not blocks and whole and split != 3
     return split >= 2 or (not blocks and K >= 2048)
 
 

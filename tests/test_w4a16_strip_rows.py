@@ -126,7 +126,9 @@ RULE = [
     (13952, 6144, 128, 33, True), (9856, 12032, 128, 64, True),     # one slice
     (3712, 11520, 0, 54, False), (3712, 11520, 128, 54, True),
     (4096, 14352, 0, 48, False), (4096, 14352, 128, 48, True),      # register-dequant kernel
-    (13824, 8208, 0, 33, False), (6144, 8208, 0, 33, False),
+    (13824, 8208, 0, 33, False), (6144, 8208, 0, 33, False), (2048, 12928, 128, 33, False),
+    (3072, 8864, 128, 41, False), (14336, 3408, 0, 47, False), (10240, 3984, 0, 34, False),
+    (8192, 3696, 128, 38, False), (9216, 3248, 128, 33, True),
     (13312, 1920, 128, 31, False), (8192, 1536, 128, 11, False),    # few strips of a long K
     (8192, 1536, 128, 24, False), (4096, 1536, 128, 24, True), (4096, 512, 0, 40, False),
     (6144, 8960, 128, 26, False), (6144, 8960, 128, 10, True),      # 140 workgroups
