@@ -27,7 +27,6 @@ PK_F32, PK_F16, PK_BF16, PK_E4M3, PK_I8, PK_U8, PK_I32 = range(7)
 _TORCH_TO_PK = {torch.float32: PK_F32, torch.float16: PK_F16, torch.bfloat16: PK_BF16}
 
 PK_OK, PK_EINVAL, PK_EUNSUPPORTED, PK_EWORKSPACE, PK_EHIP = 0, -1, -2, -3, -4
-PLAN_PACKED_B = 4  # pk_w4a16_plan's id of the packed-B GEMM
 
 KERNEL_GEMV, KERNEL_GEMM, KERNEL_SKINNY, KERNEL_GEMM_TR4 = 1, 2, 3, 4  # pk_w4a16_plan kernel ids
 
@@ -663,7 +662,7 @@ def strip_batch(M: int, K: int, N: int, group_size: int, blocks: bool) -> bool:
     plan_wgs = -(-N // 128) * split  # of the register-dequant kernel
     whole, short = group_size >= 128, 0 < group_size < 128  # groups of whole 128-row blocks
     if M > 32:
-        if kernel == PLAN_PACKED_B:
+        if kernel == KERNEL_GEMM_TR4:
             if split == 1:
                 return strips <= (1024 if whole else 512)
             return whole and split <= 3 and strips <= 512
